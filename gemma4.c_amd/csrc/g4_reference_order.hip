@@ -605,14 +605,112 @@ __device__ __forceinline__ float exact_sum_events(const float (&t)[J], uint32_t 
     return s;
 }
 
-// A hidden row of 1536 held by a block of 4 waves, lane-major: thread T
-// holds elements 6 T .. 6 T + 5 (three 8-byte loads), the layout the
-// exact-sum engine takes (thread T's J terms are terms J T .. J T + J - 1).
-// Of the block shapes that split 1536 (waves x terms a thread: 1 x 24, 2 x
-// 12, 3 x 8, 4 x 6, 6 x 4, 8 x 3, 12 x 2), 4 x 6 took the least time for a
-// fused row tail, alone (decode) and 512 rows at once (prefill): fewer terms
-// a thread shorten each wave's serial loops, more waves lengthen the block's
-// barriers.
+// ---------------------------------------------------------------------------
+// The same sequential sum for a row that fits one wave, J consecutive terms a
+// lane (lane-major): every lane runs the reference's own loop over its terms
+// from a predicted start, and the starts are corrected until each lane starts
+// bit for bit where the lane before it ended.  Lane 0 starts at the exact
+// start, so that agreement makes every lane's end -- lane 63's the row's sum --
+// the reference's, whatever the predictions were: nothing about rounding,
+// ties or binades has to be decided.
+//   start   an fp32 scan of the lanes' sums (any association)
+//   correct lane i's new start is lane i - 1's end plus the correction of lane
+//           i - 1's start: inside one binade a shift of the start shifts the
+//           end by the same amount, except where a tie rounds the other way
+//           or a step crosses into the next binade at another place
+// The first lane that disagreed gets its neighbour's end itself (the
+// corrections before it are 0), so a pass makes at least one more lane exact
+// and 64 passes always do.  Random rows of 1536 take 6 (13 at most of 200):
+// the lanes that hold a tie or a new binade, ~10 of them, half of which agree
+// by chance.  A pass is J dependent adds (~5.4 cycles each) and a 6-step lane
+// scan, ~230 cycles at J = 24, with no barrier.  Against the event table above
+// on a block of 4-8 waves (same step, before -> after): two-sum row tail of 512
+// rows 9.5 -> 8.0 us, of 37 rows 7.6 -> 6.0 us; one token's q/k/v product with
+// its two-sum tail 8.3 -> 7.6 us; q/k norms and RoPE of one token 4.7 -> 3.8 us.
+__device__ __forceinline__ float wave_prev(float x, float first) { return dpp_float<0x138, 0xf>(x, first); }
+__device__ __forceinline__ bool same_bits(float a, float b) { return __float_as_uint(a) == __float_as_uint(b); }
+
+// s_0 = 0, s_k = RN(s_{k-1} + t_k) over the wave's 64 J terms (t >= 0).
+template <int J>
+__device__ __forceinline__ float wave_chain_sum(const float (&t)[J]) {
+    const int lane = threadIdx.x & 63;
+    float part[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int j = 0; j < J; j++) part[j & 3] += t[j];
+    const float lane_sum = (part[0] + part[1]) + (part[2] + part[3]);
+    float start = wave_prev(wave_fadd_inclusive(lane_sum), 0.0f), end;
+    for (int pass = 0;; pass++) {
+        end = start;
+#pragma unroll
+        for (int j = 0; j < J; j++) end += t[j];
+        const float before = wave_prev(end, 0.0f);  // lane 0: its own exact start
+        const bool agrees = same_bits(before, start);
+        if (__ballot(!agrees) == 0 || pass == 63) break;
+        const float shift = wave_prev(wave_fadd_inclusive(agrees ? 0.0f : before - start), 0.0f);
+        start = lane == 0 ? 0.0f : before + shift;
+    }
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(end), 63));
+}
+
+// A softmax row's running sum from s: s = RN(RN(s t) + 1) at the terms flagged
+// in `fresh` (a new maximum, gemma4.c:403), s = RN(s + t) at the others; s >= 0.
+// A flagged term scales what comes before it, corrections included.
+template <int J>
+__device__ __forceinline__ float wave_chain_softmax(const float (&t)[J], uint32_t fresh, float s) {
+    const int lane = threadIdx.x & 63;
+    float fa[J], fb[J], slope = 1.0f, offset = 0.0f;  // the lane's map, an fp32 prediction
+#pragma unroll
+    for (int j = 0; j < J; j++) {
+        const bool sp = (fresh >> j) & 1;
+        fa[j] = sp ? t[j] : 1.0f;
+        fb[j] = sp ? 1.0f : t[j];
+        offset = fmaf(offset, fa[j], fb[j]);
+        slope *= fa[j];
+    }
+    const float slope_in = wave_prev(slope, 1.0f);
+    float a = slope, b = offset;
+    wave_affine_inclusive(a, b);
+    float start = fmaf(s, wave_prev(a, 1.0f), wave_prev(b, 0.0f)), end;
+    start = lane == 0 ? s : start;
+    for (int pass = 0;; pass++) {
+        end = start;
+#pragma unroll
+        for (int j = 0; j < J; j++) end = end * fa[j] + fb[j];  // s t + 1, or (s 1 exactly) + t
+        const float before = wave_prev(end, s);
+        const bool agrees = same_bits(before, start);
+        if (__ballot(!agrees) == 0 || pass == 63) break;
+        a = slope_in;
+        b = agrees ? 0.0f : before - start;
+        wave_affine_inclusive(a, b);  // b: the correction of this lane's start
+        const float shift = wave_prev(b, 0.0f);
+        // (no correction before: the neighbour's end itself)
+        start = lane == 0 ? s : shift == 0.0f ? before : fmaf(slope_in, shift, before);
+    }
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(end), 63));
+}
+
+// A 1536-wide row's sequential sum of squares by any block: every thread
+// leaves its J squares (consecutive, thread T's at J T) in the LDS row s_sq,
+// and after a barrier each wave reads the whole row, 24 terms a lane (six
+// 16-byte reads, 96 bytes apart: the 8 lanes a cycle serves hit 8 distinct
+// bank groups), and runs the chain itself -- no second barrier.
+template <int J>
+__device__ __forceinline__ float row1536_sum_squares(const float (&x)[J], float *s_sq) {
+#pragma unroll
+    for (int j = 0; j < J; j++) s_sq[J * threadIdx.x + j] = x[j] * x[j];
+    __syncthreads();
+    float t[24];
+    const float4 *row = reinterpret_cast<const float4 *>(s_sq) + 6 * (threadIdx.x & 63);
+#pragma unroll
+    for (int i = 0; i < 6; i++) {
+        const float4 f = row[i];
+        t[4 * i] = f.x, t[4 * i + 1] = f.y, t[4 * i + 2] = f.z, t[4 * i + 3] = f.w;
+    }
+    return wave_chain_sum<24>(t);
+}
+
+// A hidden row of 1536 held by a block of 4 waves: thread T holds elements
+// 6 T .. 6 T + 5 (three 8-byte loads).
 constexpr int kRowWaves = 4, kRowJ = 1536 / (64 * kRowWaves);
 __device__ __forceinline__ void load_row6(const float *row, float (&v)[kRowJ]) {
     const float2 *p = reinterpret_cast<const float2 *>(row) + 3 * threadIdx.x;
@@ -627,15 +725,6 @@ __device__ __forceinline__ void store_row6(float *row, const float (&v)[kRowJ]) 
 #pragma unroll
     for (int i = 0; i < 3; i++) p[i] = make_float2(v[2 * i], v[2 * i + 1]);
 }
-// The reference's sequential sum of squares (gemma4.c:366-368) of such a row:
-// each square rounded on its own, then the in-order fp32 chain through the
-// engine.  Every thread of the block calls it and gets the sum.
-__device__ __forceinline__ float row6_sum_squares(const float (&x)[kRowJ], EsumShared &sh) {
-    float t[kRowJ];
-#pragma unroll
-    for (int j = 0; j < kRowJ; j++) t[j] = x[j] * x[j];
-    return exact_sum_events<kRowWaves, kRowJ, false>(t, 0u, 0.0f, sh);
-}
 // y = w * (inverse * x) (gemma4.c:371-372).
 __device__ __forceinline__ void row6_scale(float (&y)[kRowJ], const float (&w)[kRowJ], float inverse,
                                            const float (&x)[kRowJ]) {
@@ -643,70 +732,47 @@ __device__ __forceinline__ void row6_scale(float (&y)[kRowJ], const float (&w)[k
     for (int j = 0; j < kRowJ; j++) y[j] = w[j] * (inverse * x[j]);
 }
 
-// The reference's sequential sum of squares (gemma4.c:366-368) of a row held
-// by a wave as xv[v] = elements 256 v + 4 lane .. + 3.  Squares are computed
-// in parallel (each is rounded on its own in the reference too); the chain
-// walks the row in order, element k = 256 v + 4 l + c living in lane l,
-// register (v, c): each square is broadcast with v_readlane into a scalar
-// register and added by the whole wave, so every lane ends with the same sum
-// and no LDS or barrier is involved.  The readlanes do not depend on the
-// chain and fill its dependent-add stalls.
-template <int V>
-__device__ __forceinline__ float row_sum_squares(const float4 (&xv)[V]) {
-    float sq[V][4];
-#pragma unroll
-    for (int v = 0; v < V; v++) {
-        sq[v][0] = xv[v].x * xv[v].x;
-        sq[v][1] = xv[v].y * xv[v].y;
-        sq[v][2] = xv[v].z * xv[v].z;
-        sq[v][3] = xv[v].w * xv[v].w;
-    }
-    float sum = 0.0f;
-#pragma unroll
-    for (int v = 0; v < V; v++)
-#pragma unroll
-        for (int l = 0; l < 64; l++)
-#pragma unroll
-            for (int c = 0; c < 4; c++)
-                sum += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(sq[v][c]), l));
-    return sum;
-}
-
-// Widths 256 * V (V = 1, 2: per-head norms of 256 and 512).  Every lane
-// holds its 4V values and weights in registers (loaded once, all loads in
-// flight); the sum is row_sum_squares.
+// Widths 256 * V (V = 1, 2: per-head norms of 256 and 512): one wave a row,
+// lane l holding elements 4 V l .. 4 V l + 4 V - 1 and their weights in
+// registers (loaded once, all loads in flight); the sum is wave_chain_sum.
 template <int V>
 __global__ __launch_bounds__(256) void k_rmsnorm_reference_v(float *out, const float *in,
                                                              const float *__restrict__ weight,
                                                              float eps, size_t rows) {
-    constexpr int W = 256 * V;
+    constexpr int W = 256 * V, J = 4 * V;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const size_t wave_row = (size_t)blockIdx.x * 4 + wave;
     if (wave_row >= rows) return;  // uniform per wave; no block-level barrier follows
-    const float4 *x4 = reinterpret_cast<const float4 *>(in + wave_row * W);
+    const float4 *x4 = reinterpret_cast<const float4 *>(in + wave_row * W) + V * lane;
     float4 xv[V], wv[V];
 #pragma unroll
-    for (int v = 0; v < V; v++) xv[v] = x4[v * 64 + lane];
+    for (int v = 0; v < V; v++) xv[v] = x4[v];
     if (weight) {
-        const float4 *w4 = reinterpret_cast<const float4 *>(weight);
+        const float4 *w4 = reinterpret_cast<const float4 *>(weight) + V * lane;
 #pragma unroll
-        for (int v = 0; v < V; v++) wv[v] = w4[v * 64 + lane];
+        for (int v = 0; v < V; v++) wv[v] = w4[v];
     } else {
 #pragma unroll
         for (int v = 0; v < V; v++) wv[v] = make_float4(1.0f, 1.0f, 1.0f, 1.0f);
     }
-    const float inverse = 1.0f / sqrtf(row_sum_squares<V>(xv) / (float)W + eps);
-    float4 *y4 = reinterpret_cast<float4 *>(out + wave_row * W);
+    float sq[J];
+#pragma unroll
+    for (int v = 0; v < V; v++) {
+        sq[4 * v] = xv[v].x * xv[v].x, sq[4 * v + 1] = xv[v].y * xv[v].y;
+        sq[4 * v + 2] = xv[v].z * xv[v].z, sq[4 * v + 3] = xv[v].w * xv[v].w;
+    }
+    const float inverse = 1.0f / sqrtf(wave_chain_sum<J>(sq) / (float)W + eps);
+    float4 *y4 = reinterpret_cast<float4 *>(out + wave_row * W) + V * lane;
 #pragma unroll
     for (int v = 0; v < V; v++)
-        y4[v * 64 + lane] = make_float4(wv[v].x * (inverse * xv[v].x), wv[v].y * (inverse * xv[v].y),
-                                        wv[v].z * (inverse * xv[v].z), wv[v].w * (inverse * xv[v].w));
+        y4[v] = make_float4(wv[v].x * (inverse * xv[v].x), wv[v].y * (inverse * xv[v].y),
+                            wv[v].z * (inverse * xv[v].z), wv[v].w * (inverse * xv[v].w));
 }
 
 // Rows of 1536 (the hidden width): one row per block (row6 layout).
 __global__ __launch_bounds__(256) void k_rmsnorm_1536(float *out, const float *in,
                                                       const float *__restrict__ weight, float eps) {
-    __shared__ EsumShared sh;
+    __shared__ __attribute__((aligned(16))) float s_sq[1536];
     const size_t row = blockIdx.x;
     float x[kRowJ], w[kRowJ];
     load_row6(in + row * 1536, x);
@@ -716,7 +782,7 @@ __global__ __launch_bounds__(256) void k_rmsnorm_1536(float *out, const float *i
 #pragma unroll
         for (int j = 0; j < kRowJ; j++) w[j] = 1.0f;
     }
-    const float inverse = 1.0f / sqrtf(row6_sum_squares(x, sh) / 1536.0f + eps);
+    const float inverse = 1.0f / sqrtf(row1536_sum_squares(x, s_sq) / 1536.0f + eps);
     float y[kRowJ];
     row6_scale(y, w, inverse, x);
     store_row6(out + row * 1536, y);
@@ -741,8 +807,9 @@ __global__ __launch_bounds__(256) void k_row_tail(const float *h, const float *_
                                                   int8_t *__restrict__ q8, float *__restrict__ qs,
                                                   float eps) {
     constexpr int W = 1536;
-    __shared__ EsumShared sh;
-    __shared__ __attribute__((aligned(16))) float s_b[QUANT ? W : 4];
+    // With two sums the first takes s_b: no wave reads it any more once the
+    // second sum's barrier is passed, so the row to quantize goes there too.
+    __shared__ __attribute__((aligned(16))) float s_b[NORM_OUT || QUANT ? W : 4], s_sq[W];
     const int T = threadIdx.x;
     const size_t row = blockIdx.x;
     float r[kRowJ], wi[kRowJ], wo[kRowJ], a[kRowJ];
@@ -753,7 +820,7 @@ __global__ __launch_bounds__(256) void k_row_tail(const float *h, const float *_
     if (NORM_OUT) load_row6(w_out, wo);
     if (ADD) {
         if (NORM_IN) {
-            const float inverse = 1.0f / sqrtf(row6_sum_squares(a, sh) / (float)W + eps);
+            const float inverse = 1.0f / sqrtf(row1536_sum_squares(a, NORM_OUT ? s_b : s_sq) / (float)W + eps);
             row6_scale(a, wi, inverse, a);
         }
 #pragma unroll
@@ -761,7 +828,7 @@ __global__ __launch_bounds__(256) void k_row_tail(const float *h, const float *_
         store_row6(residual + row * W, r);
     }
     if (NORM_OUT) {
-        const float inverse = 1.0f / sqrtf(row6_sum_squares(r, sh) / (float)W + eps);
+        const float inverse = 1.0f / sqrtf(row1536_sum_squares(r, s_sq) / (float)W + eps);
         row6_scale(r, wo, inverse, r);
     }
     if (y) store_row6(y + row * W, r);
@@ -831,7 +898,7 @@ void launch_row_tail(hipStream_t s, const float *h, const float *w_in, float *re
 constexpr int kTailGroups = 1536 / 64;
 
 // J = 24 / NW consecutive elements per thread, thread T holding J T ..
-// J T + J - 1: the lane-major layout of exact_sum_events.
+// J T + J - 1.
 template <int J>
 __device__ __forceinline__ void load_row_j(const float *row, float (&v)[J]) {
     if constexpr (J == 4) {
@@ -858,15 +925,10 @@ __device__ __forceinline__ void store_row_j(float *row, const float (&v)[J]) {
 }
 
 // y = w * (inverse * x), inverse = 1 / sqrt(sum x^2 / 1536 + eps) with the
-// sum in index order (gemma4.c:366-372); all NW waves of the block call it.
-template <int NW, int J>
-__device__ __forceinline__ void tail_rmsnorm(float (&x)[J], const float (&w)[J], float eps,
-                                             EsumShared &sh) {
-    float t[J];
-#pragma unroll
-    for (int j = 0; j < J; j++) t[j] = x[j] * x[j];
-    const float sum = exact_sum_events<NW, J, false>(t, 0u, 0.0f, sh);
-    const float inverse = 1.0f / sqrtf(sum / 1536.0f + eps);
+// sum in index order (gemma4.c:366-372); all waves of the block call it.
+template <int J>
+__device__ __forceinline__ void tail_rmsnorm(float (&x)[J], const float (&w)[J], float eps, float *s_sq) {
+    const float inverse = 1.0f / sqrtf(row1536_sum_squares(x, s_sq) / 1536.0f + eps);
 #pragma unroll
     for (int j = 0; j < J; j++) x[j] = w[j] * (inverse * x[j]);
 }
@@ -888,15 +950,16 @@ struct RowTail {
         if (NORM_IN) load_row_j<J>(tj.w_in, wi);
         if (NORM_OUT) load_row_j<J>(tj.w_out, wo);
     }
-    __device__ __forceinline__ void compute(const RowTailJob &tj, float *s_row, int *s_q8, float *s_qs,
-                                            EsumShared &sh) {
+    __device__ __forceinline__ void compute(const RowTailJob &tj, float *s_row, float *s_sq, int *s_q8,
+                                            float *s_qs) {
         if (ADD) {
-            if (NORM_IN) tail_rmsnorm<NW, J>(a, wi, tj.eps, sh);
+            // (two sums: as in k_row_tail, the first one's squares in s_row)
+            if (NORM_IN) tail_rmsnorm<J>(a, wi, tj.eps, NORM_OUT ? s_row : s_sq);
 #pragma unroll
             for (int j = 0; j < J; j++) r[j] = (r[j] + a[j]) * tj.scale;
             if (blockIdx.x == 0) store_row_j<J>(tj.res_out, r);
         }
-        if (NORM_OUT) tail_rmsnorm<NW, J>(r, wo, tj.eps, sh);
+        if (NORM_OUT) tail_rmsnorm<J>(r, wo, tj.eps, s_sq);
         store_row_j<J>(s_row, r);
         __syncthreads();
         // quantize (gemma4.c:265-279) in k_quantize's layout: 16 lanes per
@@ -927,8 +990,7 @@ void k_gemv_tail(GemvJob job, RowTailJob tj) {
     constexpr int NM = EPI == EPI_GELU_PAIR ? 2 : 1, S = EPI == EPI_PLAIN ? 1 : 4, SM = NM * S;
     constexpr int NW = W * SM, NG = kTailGroups / W;
     static_assert(NG * W == kTailGroups, "W divides 24");
-    __shared__ EsumShared sh;
-    __shared__ __attribute__((aligned(16))) float s_row[1536];
+    __shared__ __attribute__((aligned(16))) float s_row[1536], s_sq[1536];
     __shared__ int s_q8[384];
     __shared__ float s_qs[kTailGroups];
     __shared__ float s_d[SM][kTailGroups][16], s_c[SM][kTailGroups][16], s_e[NM][64];
@@ -959,7 +1021,7 @@ void k_gemv_tail(GemvJob job, RowTailJob tj) {
         wsr[u] = wscale[(g0 + u) * 16];
     }
     __builtin_amdgcn_sched_barrier(0);
-    tail.compute(tj, s_row, s_q8, s_qs, sh);
+    tail.compute(tj, s_row, s_sq, s_q8, s_qs);
 #pragma unroll
     for (int u = PRE; u < NG; u++) {
         t[u] = tiles[(size_t)(g0 + u) * 64];
@@ -2242,7 +2304,7 @@ __global__ __launch_bounds__(WAVES * 64) void k_attn_values(float *__restrict__ 
 // both written into the rings at (start_pos + t) & (cache_len - 1).  Block
 // (r, t): r < heads a query head of token t, r = heads its key, heads + 1 its
 // value.  Lane l holds elements J l .. J l + J - 1 (J = HD / 64); the sum of
-// squares is the sequential one (exact_sum_events on one wave), and element
+// squares is the sequential one (wave_chain_sum), and element
 // e's RoPE partner e + HD / 2 sits in lane l + 32, same register.
 template <int HD>
 __global__ __launch_bounds__(64) void k_qkv_finish(float *q, int heads, const float *__restrict__ q_norm,
@@ -2254,7 +2316,6 @@ __global__ __launch_bounds__(64) void k_qkv_finish(float *q, int heads, const fl
                                                    int cache_len, int start_pos,
                                                    const int *__restrict__ pos_dev) {
     constexpr int J = HD / 64;
-    __shared__ EsumShared sh;
     if (pos_dev) start_pos = *pos_dev;
     const int r = blockIdx.x, t = blockIdx.y, lane = threadIdx.x;
     const int pos = start_pos + t;
@@ -2272,7 +2333,7 @@ __global__ __launch_bounds__(64) void k_qkv_finish(float *q, int heads, const fl
     }
 #pragma unroll
     for (int i = 0; i < J; i++) sq[i] = x[i] * x[i];
-    const float inverse = 1.0f / sqrtf(exact_sum_events<1, J, false>(sq, 0u, 0.0f, sh) / (float)HD + 1e-6f);
+    const float inverse = 1.0f / sqrtf(wave_chain_sum<J>(sq) / (float)HD + 1e-6f);
 #pragma unroll
     for (int i = 0; i < J; i++) x[i] = w[i] * (inverse * x[i]);
     if (!is_v) {
