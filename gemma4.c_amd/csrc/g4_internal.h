@@ -142,8 +142,8 @@ void launch_row_tail(hipStream_t s, const float *h, const float *w_in, float *re
                      int norm_in, int add, int norm_out, int quant);
 // Position-dependent launchers take start_pos and pos_dev: when pos_dev is
 // non-null the kernels read the position from that device int instead (so a
-// captured decode graph can be replayed at every position), and the grid no
-// longer depends on the position.
+// captured decode graph can be replayed at every position up to start_pos),
+// and grids and variants are chosen for start_pos, the largest one.
 // gemma4.c:381-398 (rows of v are heads*head_dim wide)
 void launch_rope(hipStream_t s, const float *cosines, const float *sines, int pairs, float *v,
                  int heads, int head_dim, int start_pos, const int *pos_dev, size_t n);

@@ -97,14 +97,23 @@ struct Context {
     // One-token steps replay a captured graph of the whole forward pass; the
     // position is read from pos_dev.  Recaptured when the scratch buffers move
     // or the summation order changes.
-    hipGraphExec_t decode_graph = nullptr;
-    unsigned graph_generation = 0;
-    int graph_order = -1;
+    // Two of them: positions below kDecodeShort (graph 0) are served by
+    // launches that never split a softmax row over the chip, three fewer per
+    // global layer; graph 1 serves every position.
+    struct DecodeGraph {
+        hipGraphExec_t exec = nullptr;
+        unsigned generation = 0, kv_generation = 0;
+        int order = -1;
+    } decode[2];
     // The global layers' rings grow with the context (ensure_kv): a move bumps
     // kv_generation, and the captured graph (which holds the old pointers and
     // lengths) is captured again.
-    unsigned kv_generation = 0, graph_kv_generation = 0;
+    unsigned kv_generation = 0;
 };
+
+// Rows of at most kSoftmaxSplitMin values are one block's: positions 0 ..
+// kDecodeShort - 1 see no longer ones.
+constexpr int kDecodeShort = kSoftmaxSplitMin;
 
 static Context g_ctx;
 
@@ -255,7 +264,8 @@ static void free_all(Context &c) {
         if (p) (void)hipHostFree(p);
     for (hipEvent_t e : c.piece_done)
         if (e) (void)hipEventDestroy(e);
-    if (c.decode_graph) (void)hipGraphExecDestroy(c.decode_graph);
+    for (auto &g : c.decode)
+        if (g.exec) (void)hipGraphExecDestroy(g.exec);
     for (auto &lane : c.kv_written)
         for (hipEvent_t e : lane)
             if (e) (void)hipEventDestroy(e);
@@ -545,7 +555,7 @@ static int drain(Context &c) {
 // ln.tokens_dev (at positions from start_pos), as launches on ln.stream over
 // the lane's buffers.  With pos_dev non-null (n == 1) the
 // position-dependent kernels read the position from the device, so the
-// launches can be captured once and replayed at every position.
+// launches can be captured once and replayed at every position up to start_pos.
 static int enqueue_forward(Context &c, const Lane &ln, int n, int start_pos, const int *pos_dev) {
     hipStream_t s = ln.stream;
     auto matmul = [&](float *out, size_t stride, const Weight &w, int rows, bool second = false) {
@@ -771,27 +781,27 @@ static int enqueue_forward(Context &c, const Lane &ln, int n, int start_pos, con
     return G4_OK;
 }
 
-// Capture the one-token forward pass into c.decode_graph.
-static int capture_decode(Context &c) {
-    if (c.decode_graph) {
-        G4_HIP(hipGraphExecDestroy(c.decode_graph));
-        c.decode_graph = nullptr;
+// Capture the one-token forward pass for positions up to last_pos into g.
+static int capture_decode(Context &c, Context::DecodeGraph &g, int last_pos) {
+    if (g.exec) {
+        G4_HIP(hipGraphExecDestroy(g.exec));
+        g.exec = nullptr;
     }
     hipGraph_t graph = nullptr;
     G4_HIP(hipStreamBeginCapture(c.stream, hipStreamCaptureModeRelaxed));
-    const int rc = enqueue_forward(c, make_lane(c, 0), 1, 0, c.pos_dev);
+    const int rc = enqueue_forward(c, make_lane(c, 0), 1, last_pos, c.pos_dev);
     hipError_t end = hipStreamEndCapture(c.stream, &graph);
     if (rc) {
         if (graph) (void)hipGraphDestroy(graph);
         return rc;
     }
     G4_HIP(end);
-    hipError_t inst = hipGraphInstantiate(&c.decode_graph, graph, nullptr, nullptr, 0);
+    hipError_t inst = hipGraphInstantiate(&g.exec, graph, nullptr, nullptr, 0);
     (void)hipGraphDestroy(graph);
     G4_HIP(inst);
-    c.graph_generation = scratch().generation;
-    c.graph_order = order();
-    c.graph_kv_generation = c.kv_generation;
+    g.generation = scratch().generation;
+    g.order = order();
+    g.kv_generation = c.kv_generation;
     return G4_OK;
 }
 
@@ -867,10 +877,12 @@ static int forward(Context &c, const int *tokens, int n, int start_pos) {
         if (n == 1 && order() == G4_ORDER_REFERENCE) {
             *c.pos_pinned = start_pos;
             G4_HIP(hipMemcpyAsync(c.pos_dev, c.pos_pinned, sizeof(int), hipMemcpyHostToDevice, s));
-            if (!c.decode_graph || c.graph_generation != scratch().generation ||
-                c.graph_order != order() || c.graph_kv_generation != c.kv_generation)
-                G4_TRY(capture_decode(c));
-            G4_HIP(hipGraphLaunch(c.decode_graph, s));
+            const bool brief = start_pos < kDecodeShort;
+            Context::DecodeGraph &g = c.decode[brief ? 0 : 1];
+            if (!g.exec || g.generation != scratch().generation || g.order != order() ||
+                g.kv_generation != c.kv_generation)
+                G4_TRY(capture_decode(c, g, brief ? kDecodeShort - 1 : G4_MAX_CONTEXT - 1));
+            G4_HIP(hipGraphLaunch(g.exec, s));
         } else {
             G4_TRY(enqueue_forward(c, make_lane(c, 0), n, start_pos, nullptr));
         }

@@ -625,7 +625,7 @@ __device__ __forceinline__ float exact_sum_events(const float (&t)[J], uint32_t 
 // by chance.  A pass is J dependent adds (~5.4 cycles each) and a 6-step lane
 // scan, ~230 cycles at J = 24, with no barrier.  Against the event table above
 // on a block of 4-8 waves (same step, before -> after): two-sum row tail of 512
-// rows 9.5 -> 8.0 us, of 37 rows 7.6 -> 6.0 us; one token's q/k/v product with
+// rows 9.5 -> 8.0 us, of 37 rows 7.7 -> 5.7 us; one token's q/k/v product with
 // its two-sum tail 8.3 -> 7.6 us; q/k norms and RoPE of one token 4.7 -> 3.8 us.
 __device__ __forceinline__ float wave_prev(float x, float first) { return dpp_float<0x138, 0xf>(x, first); }
 __device__ __forceinline__ bool same_bits(float a, float b) { return __float_as_uint(a) == __float_as_uint(b); }
@@ -654,7 +654,9 @@ __device__ __forceinline__ float wave_chain_sum(const float (&t)[J]) {
 
 // A softmax row's running sum from s: s = RN(RN(s t) + 1) at the terms flagged
 // in `fresh` (a new maximum, gemma4.c:403), s = RN(s + t) at the others; s >= 0.
-// A flagged term scales what comes before it, corrections included.
+// A flagged term scales what comes before it, corrections included.  Window
+// rows of a decode step (512 terms) and one-wave prefill rows: with the row
+// sums above, a 37-token prompt and 16 tokens 46.5 -> 42.1 ms.
 template <int J>
 __device__ __forceinline__ float wave_chain_softmax(const float (&t)[J], uint32_t fresh, float s) {
     const int lane = threadIdx.x & 63;
@@ -1507,7 +1509,8 @@ __device__ void softmax_row_reference(float *v, int count) {
 //   v_i > before_i, e_i = expf(before_i - v_i) then, else expf(v_i - before_i)
 //   (v_0 is the starting maximum, not a term);
 //   the reference's running sum over the e_i in order (sum = sum * e + 1 at a
-//   new maximum, else sum += e) through exact_sum_events.
+//   new maximum, else sum += e): one wave's chunk, or a chunk of one value a
+//   thread, through wave_chain_softmax, larger ones through exact_sum_events.
 // Then v_i = expf(v_i - max) / sum.  Each value of the result equals the
 // one-wave kernel's bit for bit.
 
@@ -1571,9 +1574,31 @@ __device__ __forceinline__ void softmax_row_block(float *x, int count, int pad64
             fresh |= (uint32_t)is_new << j;
             before = fmaxf(before, val[j]);
         }
-        // (the engine's barriers also order these s_max reads before the next
+        // (the barriers of the sum also order these s_max reads before the next
         // chunk's writes)
-        sum = exact_sum_events<NW, J, true>(t, fresh, sum, sh);
+        if constexpr (NW == 1) {
+            sum = wave_chain_softmax<J>(t, fresh, sum);
+        } else if constexpr (J == 1) {
+            // one term a thread: the chunk through LDS, then every wave runs
+            // the chain over all of it, NW terms a lane (no wave reads s_t
+            // any more once the next chunk's s_max barrier is passed)
+            __shared__ __attribute__((aligned(16))) float s_t[C];
+            __shared__ uint64_t s_fresh[NW];
+            s_t[T] = t[0];
+            const uint64_t mask = __ballot(fresh);
+            if (lane == 0) s_fresh[wave] = mask;
+            __syncthreads();
+            float tc[NW];
+#pragma unroll
+            for (int j = 0; j < NW; j += 4) {
+                const float4 f = *reinterpret_cast<const float4 *>(&s_t[NW * lane + j]);
+                tc[j] = f.x, tc[j + 1] = f.y, tc[j + 2] = f.z, tc[j + 3] = f.w;
+            }
+            const int bit = NW * lane;  // a lane's NW flags lie in one word
+            sum = wave_chain_softmax<NW>(tc, (uint32_t)(s_fresh[bit >> 6] >> (bit & 63)) & ((1u << NW) - 1u), sum);
+        } else {
+            sum = exact_sum_events<NW, J, true>(t, fresh, sum, sh);
+        }
         run_max = chunk_max;
     }
     const int end = pad64 ? (count + 63) & ~63 : count;
@@ -1621,8 +1646,12 @@ __global__ __launch_bounds__(64 * NW) void k_softmax_block(float *__restrict__ v
                                                            SoftmaxRows spec) {
     __shared__ EsumShared sh;
     __shared__ float s_max[NW];
-    const int row = blockIdx.x;
-    softmax_row_block<NW, J>(v + (size_t)row * stride, spec.count(row), spec.pad64, sh, s_max);
+    const int row = blockIdx.x, count = spec.count(row);
+    float *x = v + (size_t)row * stride;
+    if (J > 1 && count <= 64 * NW)  // (uniform; the length is known here only)
+        softmax_row_block<NW, 1>(x, count, spec.pad64, sh, s_max);
+    else
+        softmax_row_block<NW, J>(x, count, spec.pad64, sh, s_max);
 }
 
 // Softmax of `rows` rows (attention rows (t, head) or rows of a fixed count)
@@ -2770,10 +2799,9 @@ int launch_attend_reference(hipStream_t s, float *out, const float *q, const flo
     if (heads != 8) return set_error(G4_ERR_ARG, "reference-order attention needs 8 query heads");
     if (pos_dev && n != 1) return set_error(G4_ERR_ARG, "device-side positions are for one token");
     const int last_pos = start_pos + (int)n - 1;
-    // Keys a row can see, at most; with a device-side position the bound must
-    // hold for every position, so it is the cache's.
-    const int max_keys = pos_dev ? (full ? G4_MAX_CONTEXT : G4_WINDOW)
-                                 : full ? last_pos + 1 : (last_pos + 1 < G4_WINDOW ? last_pos + 1 : G4_WINDOW);
+    // Keys a row can see, at most (with a device-side position start_pos is the
+    // largest one the launches serve).
+    const int max_keys = full ? last_pos + 1 : (last_pos + 1 < G4_WINDOW ? last_pos + 1 : G4_WINDOW);
     const size_t stride = ((size_t)max_keys + 63) & ~(size_t)63;
     const size_t score_floats = n * heads * stride;
     // decode rows that may be long: the softmax split over the CUs, its
@@ -2797,7 +2825,10 @@ int launch_attend_reference(hipStream_t s, float *out, const float *q, const flo
     // the kernel then strides over the blocks it needs)
     // blocks of kb keys
     auto key_blocks = [&](int tq, int kb) -> unsigned {
-        if (pos_dev) return full ? 512u : (unsigned)((G4_WINDOW + kb - 1) / kb);
+        if (pos_dev) {
+            const unsigned blocks = (unsigned)((max_keys + kb - 1) / kb);
+            return blocks < 512u ? blocks : 512u;
+        }
         const int tokens = (int)n < tq ? (int)n : tq;
         const int widest = full ? last_pos + 1 : G4_WINDOW - 1 + tokens;
         const int span = widest < last_pos + 1 ? widest : last_pos + 1;
