@@ -1,0 +1,317 @@
+// g4_gemm_split.hip -- W8A8 products of a few to a few dozen rows
+// (gemma4.c:192-262): the groups of a tile's K range spread over the waves of
+// a block.
+#include "g4_internal.h"
+
+namespace g4 {
+
+
+// A block computes MT 16 x 16 tiles: one 16-column weight strip by 16 MT rows.
+// Only the fold over the groups is sequential (acc = fma(dot, ws xs, acc),
+// gemma4.c:216-218); the exact int32 group dots are not.  So a phase gives
+// each of the W waves U of P = W U consecutive groups, straight from memory
+// to registers (no LDS staging, no barrier per group), leaves the dots as
+// fp32 (exact: |dot| < 2^24) in LDS, and after one barrier one thread per
+// output folds the phase's groups in order, while the next phase's loads are
+// in flight.  The tiled GEMM steps through K one group a barrier, ~205 ns
+// each whatever the number of rows.
+//
+// Operands of v_mfma_i32_16x16x64_i8, lane (l16 = l % 16, q = l / 16): the
+// activations' row l16, bytes 16 q .. + 15 of the group; of the packed weight
+// tile row l16's chunks 4 q .. 4 q + 3 (four 4-byte loads, 256 bytes a wave
+// each).  Lane l's outputs are rows 4 q + v, column l16.
+template <int W, int U, int MT>
+__global__ __launch_bounds__(64 * W) void k_gemm_split(SplitJob job, const int8_t *__restrict__ xq,
+                                                       const float *__restrict__ xs, int k, int rows,
+                                                       int row_blocks) {
+    constexpr int P = W * U, PW = P + 4, TH = 64 * W;
+    constexpr int XN = (16 * MT * P + TH - 1) / TH, WN = (16 * P + TH - 1) / TH, FN = (4 * MT + W - 1) / W;
+    __shared__ __attribute__((aligned(16))) float s_d[P * MT * 256];  // [group][tile][lane][v]
+    __shared__ __attribute__((aligned(16))) float s_w[16 * PW];       // [column][group]
+    __shared__ __attribute__((aligned(16))) float s_x[16 * MT * PW];  // [row][group]
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int q = lane >> 4, l16 = lane & 15, groups = k >> 6;
+    // Blocks go to the XCDs in turn: the row blocks of one strip are 8 ids
+    // apart, so its weights are fetched into one XCD's L2.
+    const int id = blockIdx.x, in = id % (8 * row_blocks);
+    int strip = id / (8 * row_blocks) * 8 + (in & 7), mi = 0;
+    const int m0 = (in >> 3) * 16 * MT;
+    if (strip >= job.strips) return;  // uniform: the padding to whole eights
+    while (mi + 1 < job.count && strip >= job.m[mi].strips) strip -= job.m[mi++].strips;
+    const GemvMat mat = job.m[mi];
+
+    const int *wp = reinterpret_cast<const int *>(mat.w + (size_t)strip * 16 * k) + 64 * q + l16;
+    const uint16_t *wsp = mat.ws + (size_t)strip * groups * 16;
+    const v4i *xp[MT];
+#pragma unroll
+    for (int t = 0; t < MT; t++)  // rows past the end: the last row again, not stored
+        xp[t] = reinterpret_cast<const v4i *>(xq + (size_t)min(m0 + 16 * t + l16, rows - 1) * k) + q;
+
+    v4i a[U][MT], b[U];
+    float xsv[XN];
+    uint16_t wsv[WN];
+    auto load = [&](int p0) __attribute__((always_inline)) {  // groups past the end: the last again
+#pragma unroll
+        for (int j = 0; j < XN; j++) {
+            const int i = min(tid + j * TH, 16 * MT * P - 1);
+            xsv[j] = xs[(size_t)min(m0 + i / P, rows - 1) * groups + min(p0 + i % P, groups - 1)];
+        }
+#pragma unroll
+        for (int j = 0; j < WN; j++) {
+            const int i = min(tid + j * TH, 16 * P - 1);
+            wsv[j] = wsp[min(p0 + (i >> 4), groups - 1) * 16 + (i & 15)];
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int g = min(p0 + u * W + wave, groups - 1);
+#pragma unroll
+            for (int i = 0; i < 4; i++) b[u][i] = wp[(size_t)g * 256 + 16 * i];
+#pragma unroll
+            for (int t = 0; t < MT; t++) a[u][t] = xp[t][(size_t)g * 4];
+        }
+    };
+    float acc[FN];
+#pragma unroll
+    for (int f = 0; f < FN; f++) acc[f] = 0.0f;
+    load(0);
+    for (int p0 = 0; p0 < groups; p0 += P) {
+        if (p0) __syncthreads();  // the phase before is folded
+#pragma unroll
+        for (int j = 0; j < XN; j++) {
+            const int i = tid + j * TH;
+            if (i < 16 * MT * P) s_x[i / P * PW + i % P] = xsv[j];
+        }
+#pragma unroll
+        for (int j = 0; j < WN; j++) {
+            const int i = tid + j * TH;
+            if (i < 16 * P) s_w[(i & 15) * PW + (i >> 4)] = half_bits_to_float(wsv[j]);
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++)
+#pragma unroll
+            for (int t = 0; t < MT; t++) {
+                const v4i zero = {0, 0, 0, 0};
+                const v4i d = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[u][t], b[u], zero, 0, 0, 0);
+                reinterpret_cast<float4 *>(s_d)[((u * W + wave) * MT + t) * 64 + lane] =
+                    make_float4((float)d[0], (float)d[1], (float)d[2], (float)d[3]);
+            }
+        if (p0 + P < groups) load(p0 + P);
+        __syncthreads();
+        const int count = min(P, groups - p0);
+#pragma unroll
+        for (int f = 0; f < FN; f++) {
+            const int job_at = wave + f * W;  // tile job_at / 4, rows 4 (job_at % 4) .. + 3
+            if (job_at >= 4 * MT) break;
+            const int t = job_at >> 2, m = 4 * (job_at & 3) + (lane & 3), n = lane >> 2;
+            const float *d = s_d + t * 256 + (job_at & 3) * 64 + lane;
+            const float4 *w4 = reinterpret_cast<const float4 *>(s_w + n * PW);
+            const float4 *x4 = reinterpret_cast<const float4 *>(s_x + (16 * t + m) * PW);
+            float s = acc[f];
+            int g = 0;
+#pragma unroll 3
+            for (; g + 4 <= count; g += 4) {
+                const float4 wq = w4[g >> 2], xv = x4[g >> 2];
+                s = fmaf(d[(g + 0) * MT * 256], wq.x * xv.x, s);
+                s = fmaf(d[(g + 1) * MT * 256], wq.y * xv.y, s);
+                s = fmaf(d[(g + 2) * MT * 256], wq.z * xv.z, s);
+                s = fmaf(d[(g + 3) * MT * 256], wq.w * xv.w, s);
+            }
+            for (; g < count; g++)
+                s = fmaf(d[g * MT * 256], s_w[n * PW + g] * s_x[(16 * t + m) * PW + g], s);
+            acc[f] = s;
+        }
+    }
+#pragma unroll
+    for (int f = 0; f < FN; f++) {
+        const int job_at = wave + f * W;
+        if (job_at >= 4 * MT) break;
+        const int m = m0 + 16 * (job_at >> 2) + 4 * (job_at & 3) + (lane & 3);
+        if (m < rows) mat.out[(size_t)m * job.stride[mi] + (size_t)strip * 16 + (lane >> 2)] = acc[f];
+    }
+}
+
+// The same product with a GELU epilogue, quantized output only: a block covers
+// 16 rows of 64 columns -- one quantization group -- of each of its NB
+// matrices (4 NB strips), each wave taking U groups of all of the strips a
+// phase.  After the last fold the outputs go through LDS once more, into
+// k_quantize's layout (16 lanes a group, four values a lane).
+//   EPI_GELU_PAIR  gelu(gate) * up (gemma4.c:309-331)
+//   EPI_GELU_MUL   gelu(x W^T) * mul
+template <int EPI, int W, int U>
+__global__ __launch_bounds__(64 * W) void k_gemm_split_gelu(const int8_t *__restrict__ xq,
+                                                            const float *__restrict__ xs,
+                                                            const int8_t *__restrict__ w,
+                                                            const uint16_t *__restrict__ ws, int rows,
+                                                            int n_out, int k, GemmEpilogue ep) {
+    constexpr int NB = EPI == EPI_GELU_PAIR ? 2 : 1, T = 4 * NB, P = W * U, PW = P + 4, TH = 64 * W;
+    constexpr int XN = (16 * P + TH - 1) / TH, WN = (16 * T * P + TH - 1) / TH, FN = (4 * T + W - 1) / W;
+    static_assert(TH >= 256, "one thread per four outputs of a matrix");
+    __shared__ __attribute__((aligned(16))) float s_d[P * T * 256];   // [group][strip][lane][v]
+    __shared__ __attribute__((aligned(16))) float s_w[16 * T * PW];   // [column][group]
+    __shared__ __attribute__((aligned(16))) float s_x[16 * PW];       // [row][group]
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int q = lane >> 4, l16 = lane & 15, groups = k >> 6;
+    const int m0 = blockIdx.y * 16, strip = blockIdx.x * 4;
+    const int *wp[T];
+#pragma unroll
+    for (int t = 0; t < T; t++)
+        wp[t] = reinterpret_cast<const int *>((t < 4 ? w : ep.w2) + (size_t)(strip + (t & 3)) * 16 * k) + 64 * q + l16;
+    const v4i *xp = reinterpret_cast<const v4i *>(xq + (size_t)min(m0 + l16, rows - 1) * k) + q;
+
+    v4i a[U], b[U][T];
+    float xsv[XN];
+    uint16_t wsv[WN];
+    auto load = [&](int p0) __attribute__((always_inline)) {  // groups past the end: the last again
+#pragma unroll
+        for (int j = 0; j < XN; j++) {
+            const int i = min(tid + j * TH, 16 * P - 1);
+            xsv[j] = xs[(size_t)min(m0 + i / P, rows - 1) * groups + min(p0 + i % P, groups - 1)];
+        }
+#pragma unroll
+        for (int j = 0; j < WN; j++) {
+            const int i = min(tid + j * TH, 16 * T * P - 1), t = i / (16 * P), g = min(p0 + (i / 16) % P, groups - 1);
+            const uint16_t *src = NB == 2 && t >= 4 ? ep.ws2 : ws;
+            wsv[j] = src[((size_t)(strip + (t & 3)) * groups + g) * 16 + (i & 15)];
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int g = min(p0 + u * W + wave, groups - 1);
+            a[u] = xp[(size_t)g * 4];
+#pragma unroll
+            for (int t = 0; t < T; t++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) b[u][t][i] = wp[t][(size_t)g * 256 + 16 * i];
+        }
+    };
+    float acc[FN];
+#pragma unroll
+    for (int f = 0; f < FN; f++) acc[f] = 0.0f;
+    load(0);
+    // the epilogue's multipliers arrive during the product
+    const int er = tid >> 4, ec = 4 * (tid & 15);  // (threads 0 .. 255) row and first column
+    float mulv[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (EPI == EPI_GELU_MUL && tid < 256) {
+        const float *m = ep.mul + (size_t)min(m0 + er, rows - 1) * ep.mul_stride + blockIdx.x * 64 + ec;
+#pragma unroll
+        for (int j = 0; j < 4; j++) mulv[j] = m[j];
+    }
+    for (int p0 = 0; p0 < groups; p0 += P) {
+        if (p0) __syncthreads();  // the phase before is folded
+#pragma unroll
+        for (int j = 0; j < XN; j++) {
+            const int i = tid + j * TH;
+            if (i < 16 * P) s_x[i / P * PW + i % P] = xsv[j];
+        }
+#pragma unroll
+        for (int j = 0; j < WN; j++) {
+            const int i = tid + j * TH;
+            if (i < 16 * T * P) s_w[(i / (16 * P) * 16 + (i & 15)) * PW + (i / 16) % P] = half_bits_to_float(wsv[j]);
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++)
+#pragma unroll
+            for (int t = 0; t < T; t++) {
+                const v4i zero = {0, 0, 0, 0};
+                const v4i d = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[u], b[u][t], zero, 0, 0, 0);
+                reinterpret_cast<float4 *>(s_d)[((u * W + wave) * T + t) * 64 + lane] =
+                    make_float4((float)d[0], (float)d[1], (float)d[2], (float)d[3]);
+            }
+        if (p0 + P < groups) load(p0 + P);
+        __syncthreads();
+        const int count = min(P, groups - p0);
+#pragma unroll
+        for (int f = 0; f < FN; f++) {
+            const int at = wave + f * W;  // strip at / 4, rows 4 (at % 4) .. + 3
+            if (at >= 4 * T) break;
+            const float *d = s_d + (at >> 2) * 256 + (at & 3) * 64 + lane;
+            const float4 *w4 = reinterpret_cast<const float4 *>(s_w + (16 * (at >> 2) + (lane >> 2)) * PW);
+            const float4 *x4 = reinterpret_cast<const float4 *>(s_x + (4 * (at & 3) + (lane & 3)) * PW);
+            float s = acc[f];
+            for (int g = 0; g + 4 <= count; g += 4) {  // (whole quads: groups % 8 == 0, P % 4 == 0)
+                const float4 wq = w4[g >> 2], xv = x4[g >> 2];
+                s = fmaf(d[(g + 0) * T * 256], wq.x * xv.x, s);
+                s = fmaf(d[(g + 1) * T * 256], wq.y * xv.y, s);
+                s = fmaf(d[(g + 2) * T * 256], wq.z * xv.z, s);
+                s = fmaf(d[(g + 3) * T * 256], wq.w * xv.w, s);
+            }
+            acc[f] = s;
+        }
+    }
+    __syncthreads();
+    float *s_o = s_d;  // [matrix][row][64 columns]
+#pragma unroll
+    for (int f = 0; f < FN; f++) {
+        const int at = wave + f * W;
+        if (at >= 4 * T) break;
+        const int t = at >> 2, m = 4 * (at & 3) + (lane & 3);
+        s_o[((t >> 2) * 16 + m) * 64 + (t & 3) * 16 + (lane >> 2)] = acc[f];
+    }
+    __syncthreads();
+    if (tid >= 256) return;
+    float v[4], mx = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const float gl = gelu_table_lookup(s_o[er * 64 + ec + j], ep.gelu_table, ep.gelu_size, ep.gelu_lower,
+                                           ep.gelu_upper);
+        v[j] = gl * (EPI == EPI_GELU_PAIR ? s_o[(16 + er) * 64 + ec + j] : mulv[j]);
+        mx = fmaxf(mx, fabsf(v[j]));
+    }
+#pragma unroll
+    for (int o = 8; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 16));
+    const float scale = mx / 127.0f, inverse = scale > 0.0f ? 1.0f / scale : 0.0f;
+    if (m0 + er >= rows) return;
+    char4 out;
+    out.x = (signed char)(int)rintf(v[0] * inverse);
+    out.y = (signed char)(int)rintf(v[1] * inverse);
+    out.z = (signed char)(int)rintf(v[2] * inverse);
+    out.w = (signed char)(int)rintf(v[3] * inverse);
+    *reinterpret_cast<char4 *>(ep.q_out + (size_t)(m0 + er) * n_out + blockIdx.x * 64 + ec) = out;
+    if ((tid & 15) == 0) ep.qs_out[(size_t)(m0 + er) * (n_out >> 6) + blockIdx.x] = scale;
+}
+
+// Shapes of a block, chosen by measurement (us a launch, graph replay):
+//   P = 96 groups (16 waves x 6) for up to 8 rows where they divide K's: a
+//     long K in one or two phases; 1536 x 12288 and 5 rows 9.6, against 10.3
+//     with 32; 1536 x 6144 5.5 / 5.8
+//   P = 32 (8 waves x 4) where they divide K's, else 24 (12 x 2), so that no
+//     phase runs part empty; K = 12288 and 16 rows 12.0 / 11.7, 4096 5.1 /
+//     5.5, 2048 3.8 / 4.0, 1536 3.7 / 3.4
+//   P = 4 (4 waves x 1) for fewer groups, and where K = 1536's blocks come
+//     several to a CU (more than 512): small blocks overlap each other's
+//     phases, N = 12288 and 16 rows 4.8 against 5.7 (12 x 2) and 5.3 (8 x 3);
+//     with a whole vocabulary of them, 4 x 6: 4 rows 66.7 against 74.1
+// More than one tile a block (MT = 2, 4) was no faster up to 100 rows.  The
+// VALU GEMV that took 2-8 rows before needed 81.3 us for 1536 x 12288 and 5
+// rows, 16.0 for 12288 x 1536, 10.6 for 2048 x 1536 (now 9.6, 4.4, 3.0).
+void launch_matmul_split(hipStream_t s, const SplitJob &job, const int8_t *xq, const float *xs, int k, int rows) {
+    const int groups = k / 64, rb = (rows + 15) / 16;
+    const long blocks = (long)job.strips * rb;
+    const dim3 grid((unsigned)((job.strips + 7) / 8 * 8 * rb));
+    if (groups % 96 == 0 && rows <= 8 && blocks <= 256)
+        hipLaunchKernelGGL((k_gemm_split<16, 6, 1>), grid, dim3(1024), 0, s, job, xq, xs, k, rows, rb);
+    else if (groups % 32 == 0)
+        hipLaunchKernelGGL((k_gemm_split<8, 4, 1>), grid, dim3(512), 0, s, job, xq, xs, k, rows, rb);
+    else if (groups >= 24 && blocks <= 512)
+        hipLaunchKernelGGL((k_gemm_split<12, 2, 1>), grid, dim3(768), 0, s, job, xq, xs, k, rows, rb);
+    else if (groups >= 24 && blocks > 4096)
+        hipLaunchKernelGGL((k_gemm_split<4, 6, 1>), grid, dim3(256), 0, s, job, xq, xs, k, rows, rb);
+    else
+        hipLaunchKernelGGL((k_gemm_split<4, 1, 1>), grid, dim3(256), 0, s, job, xq, xs, k, rows, rb);
+}
+
+// 96 KB of dots a block: one block a CU, so the grid has to fit the 256 CUs.
+bool launch_matmul_split_gelu(hipStream_t s, const int8_t *xq, const float *xs, const int8_t *w,
+                              const uint16_t *ws, int n_out, int k, int rows, int epi,
+                              const GemmEpilogue &ep) {
+    const dim3 grid((unsigned)(n_out / 64), (unsigned)((rows + 15) / 16));
+    if ((long)grid.x * grid.y > 256 || (k / 64) % 8) return false;
+    if (epi == EPI_GELU_MUL)
+        hipLaunchKernelGGL((k_gemm_split_gelu<EPI_GELU_MUL, 8, 3>), grid, dim3(512), 0, s, xq, xs, w, ws, rows,
+                           n_out, k, ep);
+    else
+        hipLaunchKernelGGL((k_gemm_split_gelu<EPI_GELU_PAIR, 12, 1>), grid, dim3(768), 0, s, xq, xs, w, ws, rows,
+                           n_out, k, ep);
+    return true;
+}
+
+}  // namespace g4

@@ -34,6 +34,8 @@ int set_error(int status, const char *fmt, ...);
         if (rc_) return rc_;                                                            \
     } while (0)
 
+typedef int v4i __attribute__((ext_vector_type(4)));
+
 // ---- device helpers ---------------------------------------------------------
 
 __device__ __forceinline__ float half_bits_to_float(uint16_t h) {
@@ -115,7 +117,8 @@ void layer_buffers_release();
 // gemma4.c:265-279
 void launch_quantize(hipStream_t s, int8_t *q, float *scales, const float *x, size_t groups);
 
-// gemma4.c:257-262; rows <= 8 takes the split-K GEMV, larger the MFMA GEMM.
+// gemma4.c:257-262; one row takes the GEMVs, a few (or a narrow matrix) the
+// split product (k_gemm_split), more the tiled GEMM.
 // out row stride is out_stride (>= N).
 int launch_matmul(hipStream_t s, float *out, size_t out_stride, const int8_t *xq,
                   const float *xs, const int8_t *w, const uint16_t *ws, int n_out, int k,
@@ -167,6 +170,14 @@ struct GemvJob {
     float *qs_out;
     int k;
 };
+// Up to three products of the same few-row input (k_gemm_split); out[i] has
+// row stride stride[i], strips is the sum of the matrices' strips.
+struct SplitJob {
+    GemvMat m[3];
+    size_t stride[3];
+    int count, strips;
+};
+void launch_matmul_split(hipStream_t s, const SplitJob &job, const int8_t *xq, const float *xs, int k, int rows);
 enum { EPI_PLAIN = 0, EPI_GELU_PAIR = 1, EPI_GELU_MUL = 2 };
 // The row tail that feeds a decode product (k_row_tail's arithmetic for one
 // 1536-wide row), run inside the product's launch (k_gemv_tail).
@@ -214,9 +225,9 @@ struct GemmEpilogue {
     int gn[2];
 };
 // Returns G4_ERR_ARG (and launches nothing) when the shape does not fit the
-// fused kernel (rows <= 8, K not a multiple of 512, N not of 64).
-// Up to three products of the same many-row input in one launch (K equal,
-// groups % 8 == 0, rows > 8): out[i] = x W[i]^T at out_stride[i].  Returns
+// fused kernel (one row, K not a multiple of 512, N not of 64).
+// Up to three products of the same input in one launch (K equal,
+// groups % 8 == 0): out[i] = x W[i]^T at out_stride[i].  Returns
 // G4_ERR_ARG (and launches nothing) when they do not fit.
 int launch_matmul_group(hipStream_t s, const int8_t *xq, const float *xs, int rows, int k, int count,
                         const int8_t *const *w, const uint16_t *const *ws, float *const *out,
@@ -224,6 +235,11 @@ int launch_matmul_group(hipStream_t s, const int8_t *xq, const float *xs, int ro
 int launch_matmul_gelu(hipStream_t s, const int8_t *xq, const float *xs, const int8_t *w,
                        const uint16_t *ws, int n_out, int k, int rows, int epi,
                        const GemmEpilogue &ep);
+// The same with the split product's blocks where that is faster (else false,
+// nothing launched).
+bool launch_matmul_split_gelu(hipStream_t s, const int8_t *xq, const float *xs, const int8_t *w,
+                              const uint16_t *ws, int n_out, int k, int rows, int epi,
+                              const GemmEpilogue &ep);
 
 void launch_geglu(hipStream_t s, float *gate, const float *up, int rows, int width,
                   int up_stride, const float *table, int table_size, float lower, float upper);

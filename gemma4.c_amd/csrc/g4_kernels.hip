@@ -20,7 +20,6 @@
 
 namespace g4 {
 
-typedef int v4i __attribute__((ext_vector_type(4)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 
 // ---------------------------------------------------------------------------
@@ -116,123 +115,7 @@ void launch_quantize(hipStream_t s, int8_t *q, float *scales, const float *x, si
 }
 
 // ---------------------------------------------------------------------------
-// W8A8 matmul, few rows (decode): split-K GEMV, one wave per (16-row block,
-// group range).
-//
-// A wave reads one 1024-byte tile per group with one 16-byte load per lane:
-// lane l holds chunk c = l/4 (k = 4c..4c+3) of rows 4(l%4)..4(l%4)+3.  Four
-// v_dot4_i32_i8 give the lane's partial dots; a transposing butterfly over the
-// 16 lanes that share l%4 leaves the exact int32 group dot of row
-// 4(l%4) + 2 b2 + b3 (b2, b3 = bits 2, 3 of l) in lanes 0..15.
-//
-// Memory-level parallelism: a wave issues a batch of U tiles (U KB) with the
-// activation dwords and weight scales interleaved in the order they are
-// consumed, so each group waits only for its own loads.
-//
-// Fold: acc = fma((float)dot, f32(ws) * xs, acc) over groups in ascending
-// order (gemma4.c:216-218), so results are bit-identical.  With one split per
-// block the wave folds as it goes; with several, each wave stores its exact
-// dots and k_gemv_fold (the next launch on the stream) folds all groups in
-// order -- the kernel boundary orders the two, no device-scope fences needed.
-
-// One wave's share of a one-strip GEMV: groups [g_begin, g_end) of the strip
-// at `tiles` / `wscale`, for M activation rows; `emit(g, d[M], wsr, xsv[M])`
-// gets each group's exact dots (in lanes 0..15, row `row`), raw weight scale
-// and -- with XS -- the rows' activation scales (else zeros).  Loads for a
-// batch of up to U groups are issued before any is consumed: full batches of
-// U, then one batch of the n < U left (n is the same in the whole wave; the
-// launchers pick U to suit a wave's share); slots past n reload the batch's
-// last group -- unconditional loads, so no wait at branch joins -- and are
-// not consumed.
-template <int M, int U, bool XS, typename Emit>
-__device__ __forceinline__ void gemv_strip_groups(const uint4 *tiles, const uint16_t *wscale, const int *xrow,
-                                                  const float *xs, int k, int rows, int g_begin, int g_end,
-                                                  int b2, int b3, Emit emit) {
-    const int groups = k >> 6;
-    auto batch = [&](int g0, int n) __attribute__((always_inline)) {
-        uint4 t[U];
-        int x4[U][M];
-        uint16_t wsr[U];
-        float xsv[U][M];
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            const int gu = g0 + min(u, n - 1);
-            t[u] = tiles[(size_t)gu * 64];
-#pragma unroll
-            for (int m = 0; m < M; m++) {  // rows past `rows` reread the last row (unused)
-                const int mm = min(m, rows - 1);
-                x4[u][m] = xrow[((size_t)mm * k + (size_t)gu * 64) >> 2];
-                xsv[u][m] = XS ? xs[(size_t)mm * groups + gu] : 0.0f;
-            }
-            wsr[u] = wscale[gu * 16];
-        }
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            if (u < n) {
-                int d[M];
-                gemv_group_dots<M>(t[u], x4[u], b2, b3, d);
-                emit(g0 + u, d, wsr[u], xsv[u]);
-            }
-        }
-    };
-    int g = g_begin;
-    for (; g + U <= g_end; g += U) batch(g, U);
-    if (g < g_end) batch(g, g_end - g);
-}
-
-// Batch size for a wave's share of `count` groups: the fewest batches of at
-// most `cap`, each rounded up to a multiple of 4.
-inline int gemv_batch(int count, int cap) {
-    const int batches = (count + cap - 1) / cap;
-    const int u = (count + batches - 1) / batches;
-    return (u + 3) & ~3;
-}
-
-template <int M, int U>
-__global__ __launch_bounds__(64) void k_gemv(float *__restrict__ out, size_t out_stride,
-                                             const int8_t *__restrict__ xq,
-                                             const float *__restrict__ xs,
-                                             const int8_t *__restrict__ w,
-                                             const uint16_t *__restrict__ ws, int k, int splits,
-                                             int rows, int32_t *__restrict__ dots) {
-    const int groups = k >> 6;
-    const int block = blockIdx.x / splits, split = blockIdx.x % splits;
-    const int g_begin = (int)((long)split * groups / splits);
-    const int g_end = (int)((long)(split + 1) * groups / splits);
-    const int lane = threadIdx.x;
-    const int chunk = lane >> 2, b2 = (lane >> 2) & 1, b3 = (lane >> 3) & 1;
-    const int row = 4 * (lane & 3) + 2 * b2 + b3;
-    const uint4 *tiles = reinterpret_cast<const uint4 *>(w + (size_t)block * 16 * k) + lane;
-    const uint16_t *wscale = ws + (size_t)block * groups * 16 + row;
-    const int *xrow = reinterpret_cast<const int *>(xq) + chunk;
-
-    if (splits == 1) {  // the wave folds as it goes
-        float acc[M];
-#pragma unroll
-        for (int m = 0; m < M; m++) acc[m] = 0.0f;
-        gemv_strip_groups<M, U, true>(
-            tiles, wscale, xrow, xs, k, rows, g_begin, g_end, b2, b3,
-            [&](int, const int (&d)[M], uint16_t wsr, const float (&xsv)[M]) __attribute__((always_inline)) {
-                const float wsf = half_bits_to_float(wsr);
-#pragma unroll
-                for (int m = 0; m < M; m++) acc[m] = fmaf((float)d[m], wsf * xsv[m], acc[m]);
-            });
-        if (lane < 16) {
-#pragma unroll
-            for (int m = 0; m < M; m++)
-                if (m < rows) out[(size_t)m * out_stride + (size_t)block * 16 + row] = acc[m];
-        }
-        return;
-    }
-    gemv_strip_groups<M, U, false>(
-        tiles, wscale, xrow, xs, k, rows, g_begin, g_end, b2, b3,
-        [&](int gg, const int (&d)[M], uint16_t, const float (&)[M]) __attribute__((always_inline)) {
-            if (lane < 16) {
-#pragma unroll
-                for (int m = 0; m < M; m++) dots[(((size_t)block * groups + gg) * M + m) * 16 + row] = d[m];
-            }
-        });
-}
+// W8A8 matmul, one token
 
 // The in-order fold of G groups for one output from LDS rows (16-byte
 // aligned, readable up to the next multiple of 4 plus 4): the exact dots `d`,
@@ -262,62 +145,6 @@ __device__ __forceinline__ float fold_lds_row(const float *d, const float *w, co
 }
 // LDS row length (floats) for fold_lds_row over `groups` groups
 __host__ __device__ constexpr int fold_row_floats(int groups) { return ((groups + 3) & ~3) + 4; }
-
-// Few rows, split K inside one block: W = blockDim.x / 64 waves share one
-// 16-row weight strip, wave w taking groups [w G / W, (w + 1) G / W).  Each
-// group's exact dots and weight scale go to LDS (one row per output (m, r),
-// one per weight row r), the activation scales too (loaded first, stored
-// after the weight loads); after one barrier, thread (m, r) folds its
-// output's groups in order (the reference's order, one fma each).  No second
-// kernel.  Dynamic LDS: (16 M + 16 + M) x fold_row_floats(G) floats; M x G
-// <= 4 x blockDim.x.
-template <int M, int U>
-__global__ __launch_bounds__(1024) void k_gemv_split(float *__restrict__ out, size_t out_stride,
-                                                     const int8_t *__restrict__ xq,
-                                                     const float *__restrict__ xs,
-                                                     const int8_t *__restrict__ w,
-                                                     const uint16_t *__restrict__ ws, int k,
-                                                     int rows) {
-    extern __shared__ __attribute__((aligned(16))) float s_fold[];
-    const int groups = k >> 6, waves = blockDim.x >> 6, gp = fold_row_floats(groups);
-    float *s_d = s_fold;                         // [m][r][g]
-    float *s_w = s_d + (size_t)M * 16 * gp;      // [r][g]
-    float *s_x = s_w + (size_t)16 * gp;          // [m][g]
-    const int block = blockIdx.x, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int g_begin = (int)((long)wave * groups / waves);
-    const int g_end = (int)((long)(wave + 1) * groups / waves);
-    const int chunk = lane >> 2, b2 = (lane >> 2) & 1, b3 = (lane >> 3) & 1;
-    const int row = 4 * (lane & 3) + 2 * b2 + b3;
-    const uint4 *tiles = reinterpret_cast<const uint4 *>(w + (size_t)block * 16 * k) + lane;
-    const uint16_t *wscale = ws + (size_t)block * groups * 16 + row;
-    const int *xrow = reinterpret_cast<const int *>(xq) + chunk;
-    float xsv[4];  // this thread's activation scales, stored to LDS after the weight loads
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const int i = min((int)threadIdx.x + j * (int)blockDim.x, M * groups - 1);
-        xsv[j] = M == 1 ? xs[i] : xs[(size_t)min(i / groups, rows - 1) * groups + i % groups];
-    }
-    gemv_strip_groups<M, U, false>(tiles, wscale, xrow, xs, k, rows, g_begin, g_end, b2, b3,
-                            [&](int gg, const int (&d)[M], uint16_t wsr, const float (&)[M]) __attribute__((always_inline)) {
-                                if (lane < 16) {
-#pragma unroll
-                                    for (int m = 0; m < M; m++) s_d[(m * 16 + row) * gp + gg] = (float)d[m];
-                                    s_w[row * gp + gg] = half_bits_to_float(wsr);
-                                }
-                            });
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const int i = threadIdx.x + j * blockDim.x;
-        if (i < M * groups) s_x[M == 1 ? i : (i / groups) * gp + i % groups] = xsv[j];
-    }
-    __syncthreads();
-    const int tid = threadIdx.x;
-    if (tid < 16 * M) {
-        const int m = tid >> 4, r = tid & 15;
-        const float acc = fold_lds_row(s_d + (size_t)tid * gp, s_w + (size_t)r * gp, s_x + (size_t)m * gp, groups, 0.0f);
-        if (m < rows) out[(size_t)m * out_stride + (size_t)block * 16 + r] = acc;
-    }
-}
 
 // One token (M = 1) with every CU streaming weight tiles.  A block covers one
 // 16-row strip and GB = W * U consecutive groups of it -- all of its groups
@@ -490,13 +317,14 @@ __global__ __launch_bounds__(256) void k_gemv1_fold(float *__restrict__ out, con
     if (tid < 16) out[(size_t)strip * 16 + tid] = fold_lds_row(s_d[tid], s_w[tid], s_x, groups, 0.0f);
 }
 
-// One token's product through k_gemv1 where that was measured faster than
-// k_gemv / k_gemv_split (graph replay, weights rotated past the Infinity
-// Cache): K = 1536 (24 groups) in one block of 12 waves x 2 groups (up to 384
+// One token's product through k_gemv1 where that was measured faster than the
+// split product (k_gemm_split; graph replay): K = 1536 (24 groups) in one block of 12 waves x 2 groups (up to 384
 // strips) or 8 waves x 3 groups (more); K = 2048 in 16 waves x 2 groups;
 // K = 4096 in 16 waves x 4 groups; K = 12288 split over blocks of 8 groups
-// and folded by k_gemv1_fold.  Returns false (nothing launched) for other
-// shapes (K = 256 and K = 6144 among them: the older kernels are faster).
+// and folded by k_gemv1_fold (us, against the split product: 1536 x 12288 7.8 /
+// 8.9, 1536 x 4096 4.1 / 4.3, 2048 x 1536 2.9 / 3.0).  Returns false (nothing
+// launched) for other shapes: the split product takes them (1536 x 6144 5.0 us
+// instead of the 6.0 of a VALU GEMV, 1536 x 256 2.3 instead of 2.4).
 static bool launch_gemv1(hipStream_t s, float *out, const int8_t *xq, const float *xs, const int8_t *w,
                          const uint16_t *ws, int n_out, int k) {
     const int strips = n_out / 16, groups = k / 64;
@@ -542,59 +370,6 @@ int launch_gemv_gelu(hipStream_t s, float *out, const float *a, const float *b, 
     hipLaunchKernelGGL((k_gemv1<1, 4, false, GEMV_GELU_MUL>), dim3((unsigned)(n_out / 16)), dim3(64), 0, s, out,
                        nullptr, nullptr, w, ws, k, 1, nullptr, in);
     return G4_OK;
-}
-
-// The group-ordered fold of split GEMV dots: one thread per output row.
-template <int M>
-__global__ __launch_bounds__(256) void k_gemv_fold(float *__restrict__ out, size_t out_stride,
-                                                   const int32_t *__restrict__ dots,
-                                                   const float *__restrict__ xs,
-                                                   const uint16_t *__restrict__ ws, int n_out,
-                                                   int groups, int rows) {
-    const int n = blockIdx.x * 256 + threadIdx.x;
-    if (n >= n_out) return;
-    const int block = n >> 4, r = n & 15;
-    const int32_t *d = dots + (size_t)block * groups * M * 16 + r;
-    const uint16_t *s = ws + (size_t)block * groups * 16 + r;
-    float acc[M];
-#pragma unroll
-    for (int m = 0; m < M; m++) acc[m] = 0.0f;
-    // Loads for a batch of B groups are issued before the fma chain that
-    // consumes them, so the chain is not serialized on memory latency.
-    constexpr int B = 16;
-    int g = 0;
-    for (; g + B <= groups; g += B) {
-        int dv[B][M];
-        float xv[B][M];
-        uint16_t sv[B];
-#pragma unroll
-        for (int u = 0; u < B; u++) {
-            sv[u] = s[(g + u) * 16];
-#pragma unroll
-            for (int m = 0; m < M; m++) {
-                const int mm = min(m, rows - 1);
-                dv[u][m] = d[((size_t)(g + u) * M + mm) * 16];
-                xv[u][m] = xs[(size_t)mm * groups + g + u];
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < B; u++) {
-            const float wsf = half_bits_to_float(sv[u]);
-#pragma unroll
-            for (int m = 0; m < M; m++)
-                if (m < rows) acc[m] = fmaf((float)dv[u][m], wsf * xv[u][m], acc[m]);
-        }
-    }
-    for (; g < groups; g++) {
-        const float wsf = half_bits_to_float(s[g * 16]);
-#pragma unroll
-        for (int m = 0; m < M; m++)
-            if (m < rows)
-                acc[m] = fmaf((float)d[((size_t)g * M + m) * 16], wsf * xs[(size_t)m * groups + g], acc[m]);
-    }
-#pragma unroll
-    for (int m = 0; m < M; m++)
-        if (m < rows) out[(size_t)m * out_stride + n] = acc[m];
 }
 
 // ---------------------------------------------------------------------------
@@ -1149,8 +924,9 @@ static bool small_grid(unsigned blocks) { return blocks <= 256; }
 int launch_matmul_gelu(hipStream_t s, const int8_t *xq, const float *xs, const int8_t *w,
                        const uint16_t *ws, int n_out, int k, int rows, int epi,
                        const GemmEpilogue &ep) {
-    if (rows <= 8 || k % 512 || n_out % 64 || (epi != EPI_GELU_PAIR && epi != EPI_GELU_MUL))
+    if (rows <= 1 || k % 512 || n_out % 64 || (epi != EPI_GELU_PAIR && epi != EPI_GELU_MUL))
         return set_error(G4_ERR_ARG, "fused GEMM: shape %d x %d x %d does not fit", rows, n_out, k);
+    if (launch_matmul_split_gelu(s, xq, xs, w, ws, n_out, k, rows, epi, ep)) return G4_OK;
     const dim3 grid((unsigned)(n_out / 64), (unsigned)((rows + 63) / 64));
     // the pair at K = 1536 (every gate/up): 3 LDS stages, three blocks a CU
     if (epi == EPI_GELU_PAIR && k == 1536)
@@ -1168,16 +944,33 @@ int launch_matmul_gelu(hipStream_t s, const int8_t *xq, const float *xs, const i
     return G4_OK;
 }
 
+// The split product (k_gemm_split) against the tiled GEMM: its time grows
+// with its 16-row blocks, the GEMM's is that of one block's walk through K
+// (~205 ns a group) until the grid passes the 256 CUs.  They meet near 1024
+// blocks, four a CU (us, split / GEMM): 1536 x 12288 at 100 rows (672 blocks)
+// 26 / 40, at 200 (1248) 40 / 40; 2048 x 1536 at 100 (896) 6.0 / 7.2, at 200
+// (1664) 8.9 / 7.3; 12288 x 1536 at 16 (768) 5.0 / 7.1, at 37 (2304) 9.5 /
+// 7.3.  Below 16 groups (K = 256) a GEMM block is mostly prologue: 1536 x 256
+// at 512 rows (3072 blocks) 4.7 / 4.6.
+static bool split_faster(int strips, int groups, int rows) {
+    const long blocks = (long)strips * ((rows + 15) / 16);
+    return rows <= 8 || blocks <= (groups < 16 ? 2560 : 1024);
+}
+
 int launch_matmul_group(hipStream_t s, const int8_t *xq, const float *xs, int rows, int k, int count,
                         const int8_t *const *w, const uint16_t *const *ws, float *const *out,
                         const size_t *out_stride, const int *n_out) {
-    if (rows <= 8 || k % 512 || count < 1 || count > 3)
+    if (rows < 1 || k % 512 || count < 1 || count > 3)
         return set_error(G4_ERR_ARG, "grouped GEMM: %d products of %d rows x K %d do not fit", count, rows, k);
     GemmEpilogue ep{};
+    SplitJob job{};
     unsigned cols = 0;
     for (int i = 0; i < count; i++) {
         if (n_out[i] <= 0 || n_out[i] % 16)
             return set_error(G4_ERR_ARG, "grouped GEMM: N %d is not a multiple of 16", n_out[i]);
+        job.m[i] = GemvMat{w[i], ws[i], out[i], n_out[i] / 16};
+        job.stride[i] = out_stride[i];
+        job.strips += n_out[i] / 16;
         ep.cols[i] = (n_out[i] / 16 + 3) / 4;
         cols += (unsigned)ep.cols[i];
         if (i) {
@@ -1187,6 +980,11 @@ int launch_matmul_group(hipStream_t s, const int8_t *xq, const float *xs, int ro
             ep.gstride[i - 1] = out_stride[i];
             ep.gn[i - 1] = n_out[i];
         }
+    }
+    job.count = count;
+    if (split_faster(job.strips, k / 64, rows)) {
+        launch_matmul_split(s, job, xq, xs, k, rows);
+        return G4_OK;
     }
     const dim3 grid(cols, (unsigned)((rows + 63) / 64));
     if (small_grid(grid.x * grid.y))
@@ -1202,100 +1000,35 @@ int launch_matmul(hipStream_t s, float *out, size_t out_stride, const int8_t *xq
                   const int8_t *w, const uint16_t *ws, int n_out, int k, int rows) {
     if (rows <= 0) return G4_OK;
     const int blocks = n_out / 16, groups = k / 64;
-    if (rows > 8) {
-        const unsigned mb = (unsigned)((rows + 63) / 64);
-        const dim3 grid((unsigned)((blocks + 3) / 4), mb), grid48((unsigned)(blocks / 3), mb);
-        GemmEpilogue ep{};
-        ep.cols[0] = (int)grid.x;
-        if (groups % 8 == 0 && blocks % 3 == 0 && grid.x * grid.y < 256 && grid48.x * grid48.y <= 256) {
-            // 48-wide tiles fill more of the 256 CUs (N = 1536 at 512 rows: 256 blocks, not 192)
-            ep.cols[0] = (int)grid48.x;
-            hipLaunchKernelGGL((k_gemm_dma<EPI_PLAIN, 6, 3>), grid48, dim3(384), 0, s, out, out_stride, xq,
-                               xs, w, ws, rows, n_out, k, ep);
-        } else if (groups % 8 == 0 && small_grid(grid.x * grid.y))
-            hipLaunchKernelGGL((k_gemm_dma<EPI_PLAIN, 8>), grid, dim3(512), 0, s, out,
-                               out_stride, xq, xs, w, ws, rows, n_out, k, ep);
-        else if (groups % 8 == 0)
-            hipLaunchKernelGGL((k_gemm_dma<EPI_PLAIN, 4>), grid, dim3(256), 0, s, out, out_stride, xq,
-                               xs, w, ws, rows, n_out, k, ep);
-        else  // K not a multiple of 512 (the per-layer-embedding projection, K = 256):
-              // the register-staged kernel, two groups per barrier
-            hipLaunchKernelGGL((k_gemm<64, 2>), dim3((unsigned)((blocks + 3) / 4), mb), dim3(256), 0, s,
-                               out, out_stride, xq, xs, w, ws, rows, n_out, k);
-        return G4_OK;
-    }
     if (rows == 1 && launch_gemv1(s, out, xq, xs, w, ws, n_out, k)) return G4_OK;
-    const int m_pad = rows <= 1 ? 1 : rows <= 2 ? 2 : rows <= 4 ? 4 : 8;
-    // Enough waves to keep ~16 KB in flight on every CU: aim for >= 2048 waves,
-    // each covering at least 8 groups (8 KB of weights).
-    int splits = 1;
-    if (blocks < 2048) {
-        splits = (2048 + blocks - 1) / blocks;
-        const int max_splits = groups / 8 > 0 ? groups / 8 : 1;
-        if (splits > max_splits) splits = max_splits;
-    }
-    // Split K inside one block when the per-group dots fit in LDS: no fold kernel.
-    const int split_waves = splits < 16 ? splits : 16;
-    const size_t fold_lds = (size_t)(16 * m_pad + 16 + m_pad) * fold_row_floats(groups) * sizeof(float);
-    if (splits > 1 && fold_lds <= 64 * 1024 && m_pad * groups <= 4 * 64 * split_waves) {
-        // one batch of loads per wave where the registers allow it
-        const int per_wave = (groups + split_waves - 1) / split_waves;
-#define G4_GEMV_SPLIT(MM, UU)                                                                   \
-    hipLaunchKernelGGL((k_gemv_split<MM, UU>), dim3((unsigned)blocks), dim3(64 * split_waves), fold_lds, s, \
-                       out, out_stride, xq, xs, w, ws, k, rows)
-        switch (m_pad) {
-        case 1:  // batches of at most 12 (16 would spill with 16 waves a block)
-            switch (gemv_batch(per_wave, 12)) {
-            case 4: G4_GEMV_SPLIT(1, 4); break;
-            case 8: G4_GEMV_SPLIT(1, 8); break;
-            default: G4_GEMV_SPLIT(1, 12); break;
-            }
-            break;
-        case 2: G4_GEMV_SPLIT(2, 8); break;
-        case 4: G4_GEMV_SPLIT(4, 4); break;
-        default: G4_GEMV_SPLIT(8, 4); break;
-        }
-#undef G4_GEMV_SPLIT
+    if (split_faster(blocks, groups, rows)) {
+        SplitJob job{};
+        job.m[0] = GemvMat{w, ws, out, blocks};
+        job.stride[0] = out_stride;
+        job.count = 1;
+        job.strips = blocks;
+        launch_matmul_split(s, job, xq, xs, k, rows);
         return G4_OK;
     }
-    int32_t *dots = nullptr;
-    if (splits > 1) {
-        const size_t need = (size_t)n_out * groups * m_pad * sizeof(int32_t);
-        int rc = scratch_reserve(need, 0);
-        if (rc) return rc;
-        dots = scratch().dots;
-    }
-    dim3 grid((unsigned)(blocks * splits));
-#define G4_GEMV(MM, UU)                                                                        \
-    hipLaunchKernelGGL((k_gemv<MM, UU>), grid, dim3(64), 0, s, out, out_stride, xq, xs, w, ws, \
-                       k, splits, rows, dots)
-    switch (m_pad) {
-    case 1:
-        switch (gemv_batch((groups + splits - 1) / splits, 16)) {
-        case 4: G4_GEMV(1, 4); break;
-        case 8: G4_GEMV(1, 8); break;
-        case 12: G4_GEMV(1, 12); break;
-        default: G4_GEMV(1, 16); break;
-        }
-        break;
-    case 2: G4_GEMV(2, 8); break;
-    case 4: G4_GEMV(4, 4); break;
-    default: G4_GEMV(8, 4); break;
-    }
-#undef G4_GEMV
-    if (splits > 1) {
-        dim3 fgrid((unsigned)((n_out + 255) / 256));
-#define G4_FOLD(MM)                                                                            \
-    hipLaunchKernelGGL((k_gemv_fold<MM>), fgrid, dim3(256), 0, s, out, out_stride, dots, xs, ws, \
-                       n_out, groups, rows)
-        switch (m_pad) {
-        case 1: G4_FOLD(1); break;
-        case 2: G4_FOLD(2); break;
-        case 4: G4_FOLD(4); break;
-        default: G4_FOLD(8); break;
-        }
-#undef G4_FOLD
-    }
+    const unsigned mb = (unsigned)((rows + 63) / 64);
+    const dim3 grid((unsigned)((blocks + 3) / 4), mb), grid48((unsigned)(blocks / 3), mb);
+    GemmEpilogue ep{};
+    ep.cols[0] = (int)grid.x;
+    if (groups % 8 == 0 && blocks % 3 == 0 && grid.x * grid.y < 256 && grid48.x * grid48.y <= 256) {
+        // 48-wide tiles fill more of the 256 CUs (N = 1536 at 512 rows: 256 blocks, not 192)
+        ep.cols[0] = (int)grid48.x;
+        hipLaunchKernelGGL((k_gemm_dma<EPI_PLAIN, 6, 3>), grid48, dim3(384), 0, s, out, out_stride, xq,
+                           xs, w, ws, rows, n_out, k, ep);
+    } else if (groups % 8 == 0 && small_grid(grid.x * grid.y))
+        hipLaunchKernelGGL((k_gemm_dma<EPI_PLAIN, 8>), grid, dim3(512), 0, s, out,
+                           out_stride, xq, xs, w, ws, rows, n_out, k, ep);
+    else if (groups % 8 == 0)
+        hipLaunchKernelGGL((k_gemm_dma<EPI_PLAIN, 4>), grid, dim3(256), 0, s, out, out_stride, xq,
+                           xs, w, ws, rows, n_out, k, ep);
+    else  // K not a multiple of 512 (the per-layer-embedding projection, K = 256):
+          // the register-staged kernel, two groups per barrier
+        hipLaunchKernelGGL((k_gemm<64, 2>), dim3((unsigned)((blocks + 3) / 4), mb), dim3(256), 0, s,
+                           out, out_stride, xq, xs, w, ws, rows, n_out, k);
     return G4_OK;
 }
 

@@ -105,7 +105,7 @@ extern "C" int g4_attention_layer(void *stream, float *hidden, size_t n, int sta
     const float *cs = (const float *)cosines.data, *sn = (const float *)sines.data;
     // gemma4.c:425-426, 435-436: the queries, and the new keys and values
     launch_quantize(s, b.q8, b.qs, hidden, n * (G4_HIDDEN / 64));
-    if (writes && n > 8) {  // one launch for the three products of the same rows
+    if (writes) {  // one launch for the three products of the same rows
         const int8_t *w[3] = {(const int8_t *)q.data, (const int8_t *)k.data, (const int8_t *)v.data};
         const uint16_t *ws[3] = {q.scales, k.scales, v.scales};
         float *out[3] = {b.aux, b.k_new, b.v_new};
@@ -114,10 +114,6 @@ extern "C" int g4_attention_layer(void *stream, float *hidden, size_t n, int sta
         G4_TRY(launch_matmul_group(s, b.q8, b.qs, (int)n, G4_HIDDEN, 3, w, ws, out, strides, ns));
     } else {
         G4_TRY(launch_matmul(s, b.aux, qw, b.q8, b.qs, (const int8_t *)q.data, q.scales, qw, G4_HIDDEN, (int)n));
-        if (writes) {
-            G4_TRY(launch_matmul(s, b.k_new, hd, b.q8, b.qs, (const int8_t *)k.data, k.scales, hd, G4_HIDDEN, (int)n));
-            G4_TRY(launch_matmul(s, b.v_new, hd, b.q8, b.qs, (const int8_t *)v.data, v.scales, hd, G4_HIDDEN, (int)n));
-        }
     }
     // gemma4.c:427-428, 437-440: norms and RoPE, the new rows into the ring
     if (order() == G4_ORDER_REFERENCE) {

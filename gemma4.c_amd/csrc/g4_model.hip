@@ -638,7 +638,7 @@ static int enqueue_forward(Context &c, const Lane &ln, int n, int start_pos, con
                                          : tail_job(ln.hidden, c.layers[l - 1].post_ple_ln,
                                                     c.layers[l - 1].layer_scalar, L.input_ln);
             G4_TRY(launch_gemv_tail(s, job, EPI_PLAIN, tj, l == 0 ? 3 : 1));
-        } else if (L.k.data && n > 8 && G4_HIDDEN % 512 == 0) {
+        } else if (L.k.data && n > 1 && G4_HIDDEN % 512 == 0) {
             // q, k and v read the same rows: one launch fills the chip
             const int8_t *w[3] = {L.q.data, L.k.data, L.v.data};
             const uint16_t *ws[3] = {L.q.scales, L.k.scales, L.v.scales};
@@ -686,7 +686,7 @@ static int enqueue_forward(Context &c, const Lane &ln, int n, int start_pos, con
         }
         // many rows: gate and up in one GEMM whose epilogue applies geglu and
         // quantizes (into q8b)
-        const bool gemm_fused = n > 8;
+        const bool gemm_fused = n > 1;
         auto gelu_epilogue = [&]() {
             GemmEpilogue ep{};
             ep.gelu_table = c.gelu;

@@ -1,0 +1,60 @@
+"""The split product (a K range's groups over the waves of a block): every
+block shape at the edges of its rows, strips and phases, bit for bit against
+the oracle; and its GELU epilogues through whole passes of few tokens."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from conftest import random_weight, rng
+from helpers import DeviceWeight, HostWeight
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("rows,n,k", [
+    (1, 16, 64), (2, 48, 64 * 3), (16, 16, 64 * 5),          # 4 x 1: one strip, part phases
+    (17, 400, 64 * 23), (33, 8192, 1536),                    # 4 x 1: ragged rows; many blocks of K = 1536
+    (3, 272, 1536), (31, 48, 64 * 25), (64, 1536, 64 * 49),  # 12 x 2: strips not a multiple of 8, a last group alone
+    (1, 1536, 6144), (8, 1536, 12288), (5, 16, 6144),        # 16 x 6
+    (9, 1536, 12288), (15, 48, 2048), (100, 1536, 4096),     # 8 x 4
+    (2, 70000 // 16 * 16, 1536),                             # 4 x 6: more blocks than 16 a CU
+    (170, 1536, 6144), (171, 1536, 2048), (512, 1536, 256),  # either side of the tiled GEMM's line
+])
+def test_split_product_bitexact(pkg, g4lib, torch_gpu, oracle_lib, rows, n, k):
+    torch, ok = torch_gpu, oracle_lib.Kernels()
+    g = rng(rows * 31 + n + k)
+    w, s = random_weight(g, n, k)
+    hw = HostWeight(pkg, w, s)
+    dw = DeviceWeight(pkg, torch, hw)
+    xq, xs = ok.quantize(g.standard_normal((rows, k)).astype(np.float32))
+    xs[rows // 2, k // 128] = np.inf  # one row's alone: nothing of it in its neighbours
+    xqd, xsd = torch.from_numpy(xq).cuda(), torch.from_numpy(xs).cuda()
+    out = torch.full((rows + 1, n), 7.5, device="cuda")  # a row past the end stays as it was
+    pkg.check(g4lib.g4_matmul_int8(None, out.data_ptr(), xqd.data_ptr(), xsd.data_ptr(), dw.record, rows))
+    torch.cuda.synchronize()
+    out = out.cpu().numpy()
+    assert np.array_equal(out[:rows], ok.matmul(xq, xs, hw.record, n), equal_nan=True)
+    assert (out[rows] == 7.5).all()
+
+
+@pytest.mark.parametrize("chunks", [(2, 5), (8, 9), (16, 17)])
+def test_few_token_passes(pkg, g4lib, image, oracle_lib, chunks):
+    """Gate and up, and the per-layer-embedding gate, in 16-row blocks and past them."""
+    pkg.check(g4lib.g4_init(image.records, 0))
+    cpu = oracle_lib.Model(image)
+    try:
+        pos = 0
+        for n in chunks:
+            tokens = rng(100 + n).integers(0, pkg.VOCAB, n).astype(np.int32)
+            pkg.check(g4lib.g4_forward(tokens.ctypes.data, n, pos))
+            cpu.forward(tokens, pos)
+            pos += n
+            out = np.empty(pkg.VOCAB, np.float32)
+            for r in (0, n - 1):
+                pkg.check(g4lib.g4_logits(r, out.ctypes.data))
+                assert np.array_equal(out, cpu.logits(r)), (n, r)
+    finally:
+        cpu.close()
+        g4lib.g4_shutdown()
