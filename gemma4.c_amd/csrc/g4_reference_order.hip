@@ -25,6 +25,8 @@
 //   Checked against the host libm on every input of its main path.
 #include <math.h>
 
+#include <type_traits>
+
 #include "g4_internal.h"
 
 namespace g4 {
@@ -630,24 +632,24 @@ __device__ __forceinline__ float exact_sum_events(const float (&t)[J], uint32_t 
 __device__ __forceinline__ float wave_prev(float x, float first) { return dpp_float<0x138, 0xf>(x, first); }
 __device__ __forceinline__ bool same_bits(float a, float b) { return __float_as_uint(a) == __float_as_uint(b); }
 
-// s_0 = 0, s_k = RN(s_{k-1} + t_k) over the wave's 64 J terms (t >= 0).
+// s_0 = s >= 0, s_k = RN(s_{k-1} + t_k) over the wave's 64 J terms (t >= 0).
 template <int J>
-__device__ __forceinline__ float wave_chain_sum(const float (&t)[J]) {
+__device__ __forceinline__ float wave_chain_sum(const float (&t)[J], float s = 0.0f) {
     const int lane = threadIdx.x & 63;
     float part[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int j = 0; j < J; j++) part[j & 3] += t[j];
     const float lane_sum = (part[0] + part[1]) + (part[2] + part[3]);
-    float start = wave_prev(wave_fadd_inclusive(lane_sum), 0.0f), end;
+    float start = s + wave_prev(wave_fadd_inclusive(lane_sum), 0.0f), end;
     for (int pass = 0;; pass++) {
         end = start;
 #pragma unroll
         for (int j = 0; j < J; j++) end += t[j];
-        const float before = wave_prev(end, 0.0f);  // lane 0: its own exact start
+        const float before = wave_prev(end, s);  // lane 0: its own exact start
         const bool agrees = same_bits(before, start);
         if (__ballot(!agrees) == 0 || pass == 63) break;
         const float shift = wave_prev(wave_fadd_inclusive(agrees ? 0.0f : before - start), 0.0f);
-        start = lane == 0 ? 0.0f : before + shift;
+        start = lane == 0 ? s : before + shift;
     }
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(end), 63));
 }
@@ -1517,7 +1519,7 @@ __device__ void softmax_row_reference(float *v, int count) {
 // Which values a row holds: a fixed count, or an attention row (t, head)
 // whose visible keys follow from the position.  pad64: the row's stride
 // leaves room to round the count up to a multiple of 64, and the values
-// between are written as 0 (the decode P.V kernel reads whole 64-key tiles).
+// between are written as -0 (the decode P.V kernel reads whole 64-key tiles).
 struct SoftmaxRows {
     int heads, full, start_pos, fixed_count;
     const int *pos_dev;
@@ -1603,7 +1605,7 @@ __device__ __forceinline__ void softmax_row_block(float *x, int count, int pad64
     }
     const int end = pad64 ? (count + 63) & ~63 : count;
     if (count <= C) {  // one chunk: a value a lane at a time (short rows skip lanes)
-        for (int i = T; i < end; i += 64 * NW) x[i] = i < count ? expf_libm(x[i] - run_max) / sum : 0.0f;
+        for (int i = T; i < end; i += 64 * NW) x[i] = i < count ? expf_libm(x[i] - run_max) / sum : -0.0f;
         return;
     }
     // Longer rows chunk by chunk, a chunk's loads all issued first (a value a
@@ -1629,7 +1631,7 @@ __device__ __forceinline__ void softmax_row_block(float *x, int count, int pad64
             float o[4];
 #pragma unroll
             for (int e = 0; e < 4 && j + e < J; e++)
-                o[e] = i + e < count ? expf_libm(v[j + e] - run_max) / sum : 0.0f;
+                o[e] = i + e < count ? expf_libm(v[j + e] - run_max) / sum : -0.0f;
             if (J % 4 == 0 && wide && i + 3 < end) {
                 *reinterpret_cast<float4 *>(x + i) = make_float4(o[0], o[1], o[2], o[3]);
             } else {
@@ -1677,7 +1679,7 @@ static void launch_softmax_block(hipStream_t s, float *v, size_t stride, int max
 //     block holding the row's last value writes the row's maximum;
 //   k_softmax_sum (a block per row): the reference's running sum over those
 //     terms in order (exact_sum_events, which is exact whatever the chunks);
-//   k_softmax_norm (every CU): v_i = expf(v_i - max) / sum, and the zeros up
+//   k_softmax_norm (every CU): v_i = expf(v_i - max) / sum, and -0 up
 //     to the tile end.
 // A row of at most kSplitMin values (known on the device only, with a
 // device-side position) is done whole by k_softmax_sum's block, as
@@ -2124,7 +2126,7 @@ __global__ __launch_bounds__(256) void k_softmax_norm(float *__restrict__ v, siz
     if (count <= kSplitMin || lo >= end) return;
     const float mx = w.max[row], sum = w.sum[row];
     float *x = v + (size_t)row * stride;
-    for (int i = lo + (int)threadIdx.x; i < end; i += 256) x[i] = i < count ? expf_libm(x[i] - mx) / sum : 0.0f;
+    for (int i = lo + (int)threadIdx.x; i < end; i += 256) x[i] = i < count ? expf_libm(x[i] - mx) / sum : -0.0f;
 }
 
 // The three launches over `rows` rows; `work` holds softmax_split_bytes(rows, stride).
@@ -2137,40 +2139,115 @@ static void launch_softmax_split(hipStream_t s, float *v, size_t stride, Softmax
     hipLaunchKernelGGL(k_softmax_norm, dim3(kSplitBlocks, rows), dim3(256), 0, s, v, stride, spec, w);
 }
 
-// Attention probabilities of every (token, head) row of a prefill pass, a
-// block of NW waves per row running softmax_row_block in chunks of 512 NW
-// values: one wave for rows of at most a window (a 64-value step at a time
-// took 20.7 against 16.6 us for 4096 rows at the start of a prefill), four
-// for the long rows of a global layer deep in a prefill (181 against 249 us
-// for 4096 rows of 7681-8192 values).
+// One row longer than a window by one wave, in chunks of 64 J values, lane l
+// holding J consecutive ones; the sum as wave_chain_sum from the chunk
+// before's.  A new maximum is rare past the first chunk: without one a chunk's
+// terms are expf(v - max) and its sum plain adds.  Then v = expf(v - max) /
+// sum, 16 bytes a lane.
+template <int J>
+__device__ __forceinline__ void softmax_row_wave(float *x, int count, int end) {
+    constexpr int C = 64 * J;
+    const int lane = threadIdx.x & 63;
+    float run_max = x[0], sum = 1.0f;  // gemma4.c:401
+    float next[J];
+    auto load = [&](int base) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < J; j += 4) {
+            const int i = base + J * lane + j;
+            if (i + 3 < count) {
+                const float4 f = *reinterpret_cast<const float4 *>(x + i);
+                next[j] = f.x, next[j + 1] = f.y, next[j + 2] = f.z, next[j + 3] = f.w;
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; e++) next[j + e] = i + e < count ? x[i + e] : -INFINITY;  // a zero term
+            }
+        }
+    };
+    load(0);
+    if (lane == 0) next[0] = -INFINITY;  // v_0 is the starting maximum, not a term
+    for (int base = 0; base < count; base += C) {
+        float val[J], t[J], m = -INFINITY;
+#pragma unroll
+        for (int j = 0; j < J; j++) {
+            val[j] = next[j];
+            m = fmaxf(m, val[j]);
+        }
+        if (base + C < count) load(base + C);
+        if (__ballot(m > run_max) == 0) {
+#pragma unroll
+            for (int j = 0; j < J; j++) t[j] = expf_libm(val[j] - run_max);
+            sum = wave_chain_sum<J>(t, sum);
+            continue;
+        }
+        const float incl = wave_max_scan(m);
+        float before = fmaxf(run_max, dpp_float<0x138, 0xf>(incl, -INFINITY));  // lanes below
+        uint32_t fresh = 0;
+#pragma unroll
+        for (int j = 0; j < J; j++) {
+            const bool is_new = val[j] > before;
+            t[j] = is_new ? expf_libm(before - val[j]) : expf_libm(val[j] - before);
+            fresh |= (uint32_t)is_new << j;
+            before = fmaxf(before, val[j]);
+        }
+        sum = wave_chain_softmax<J>(t, fresh, sum);
+        run_max = fmaxf(run_max, __int_as_float(__builtin_amdgcn_readlane(__float_as_int(incl), 63)));
+    }
+    for (int base = 0; base < end; base += 1024) {
+        float4 v[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {  // (the row's stride is a multiple of 64: in bounds)
+            const int i = base + 256 * u + 4 * lane;
+            v[u] = i < count ? *reinterpret_cast<const float4 *>(x + i) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        }
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const int i = base + 256 * u + 4 * lane;
+            float o[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
+#pragma unroll
+            for (int e = 0; e < 4; e++) o[e] = i + e < count ? expf_libm(o[e] - run_max) / sum : -0.0f;
+            if (i + 3 < end) {
+                *reinterpret_cast<float4 *>(x + i) = make_float4(o[0], o[1], o[2], o[3]);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    if (i + e < end) x[i + e] = o[e];
+            }
+        }
+    }
+}
+
+// Attention probabilities of every (token, head) row of a prefill pass, NW
+// waves a row.  Rows of at most a window take one wave and the fewest terms a
+// lane that hold them in one chunk (a causal chunk's early tokens have short
+// rows; 512 tokens x 8 heads from position 0: 14.2 against 15.6 us with 8
+// terms a lane).  Longer ones take four waves in chunks of 2048, or, where
+// there are several rows a SIMD to hide each other's chains, one wave each
+// (softmax_row_wave; launch_attend_reference has both sides' times).
+// pad64: the values up to the next multiple of 64 are written as -0.
 template <int NW>
-__global__ __launch_bounds__(64 * NW) void k_attn_softmax_reference(float *__restrict__ scores,
-                                                                    int heads, int full, int start_pos,
-                                                                    const int *__restrict__ pos_dev,
-                                                                    size_t stride) {
+__global__ __launch_bounds__(64 * NW) void k_attn_softmax_reference(float *__restrict__ scores, int heads,
+                                                                    int full, int start_pos, size_t stride,
+                                                                    int pad64) {
     __shared__ EsumShared sh;
     __shared__ float s_max[NW];
-    if (pos_dev) start_pos = *pos_dev;
     // last token first: rows grow with the token (causal), so the longest
     // start first and the short ones fill in behind them
     const int h = blockIdx.x, t = gridDim.y - 1 - blockIdx.y;
     const int pos = start_pos + t, keys = pos + 1 - first_visible(pos, full);
     float *row = scores + ((size_t)t * heads + h) * stride;
     if constexpr (NW == 1) {
-        // the fewest terms a lane that hold the row in one chunk: the engine's
-        // per-term phases shrink with them (a causal chunk's early tokens have
-        // short rows; 512 tokens x 8 heads from position 0: 14.2 against
-        // 15.6 us with 8 terms a lane)
         if (keys <= 64)
-            softmax_row_block<1, 1>(row, keys, 0, sh, s_max);
+            softmax_row_block<1, 1>(row, keys, pad64, sh, s_max);
         else if (keys <= 128)
-            softmax_row_block<1, 2>(row, keys, 0, sh, s_max);
+            softmax_row_block<1, 2>(row, keys, pad64, sh, s_max);
         else if (keys <= 256)
-            softmax_row_block<1, 4>(row, keys, 0, sh, s_max);
+            softmax_row_block<1, 4>(row, keys, pad64, sh, s_max);
+        else if (keys <= 512)
+            softmax_row_block<1, 8>(row, keys, pad64, sh, s_max);
         else
-            softmax_row_block<1, 8>(row, keys, 0, sh, s_max);
+            softmax_row_wave<16>(row, keys, pad64 ? (keys + 63) & ~63 : keys);
     } else {
-        softmax_row_block<NW, 8>(row, keys, 0, sh, s_max);
+        softmax_row_block<NW, 8>(row, keys, pad64, sh, s_max);
     }
 }
 
@@ -2194,18 +2271,21 @@ __global__ __launch_bounds__(64) void k_softmax_rows(float *values, int count, s
 // each wave's probabilities [head][key] beside them (rows padded by 4 floats,
 // so the 4 heads one read serves sit on different banks); both are prefetched
 // DEPTH tiles ahead in registers with unconditional loads.
+//
+// For passes of some tens of tokens: a token's two 4x4x1 chains step a key in
+// ~54 cycles where k_attn_values' 16x16x1 takes ~75, and its waves are too few
+// there to hide that (launch_attend_reference).
 template <int HD, int WAVES, int DEPTH>
-__global__ __launch_bounds__(WAVES * 64) void k_attn_values(float *__restrict__ out,
-                                                            const float *__restrict__ probs,
-                                                            const float *__restrict__ value_cache,
-                                                            int cache_len, int full, int start_pos,
-                                                            int n, const int *__restrict__ pos_dev,
-                                                            size_t stride, int8_t *__restrict__ q8,
-                                                            float *__restrict__ qs) {
+__global__ __launch_bounds__(WAVES * 64) void k_attn_values_staged(float *__restrict__ out,
+                                                                   const float *__restrict__ probs,
+                                                                   const float *__restrict__ value_cache,
+                                                                   int cache_len, int full, int start_pos,
+                                                                   int n, size_t stride,
+                                                                   int8_t *__restrict__ q8,
+                                                                   float *__restrict__ qs) {
     typedef float v4 __attribute__((ext_vector_type(4)));
     constexpr int HEADS = 8;
     constexpr int THREADS = WAVES * 64;
-    if (pos_dev) start_pos = *pos_dev;
     constexpr int F4 = 64 * 64 / 4 / THREADS;   // float4 per thread per tile
     __shared__ __attribute__((aligned(16))) float s_v[64][64 + 4];
     __shared__ __attribute__((aligned(16))) float s_p[WAVES][HEADS][64 + 4];
@@ -2326,6 +2406,186 @@ __global__ __launch_bounds__(WAVES * 64) void k_attn_values(float *__restrict__ 
     }
 }
 
+// f(integral_constant<0>) .. f(integral_constant<N - 1>)
+template <int N, int I = 0, typename F>
+__device__ __forceinline__ void unroll_for(F f) {
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>{});
+        unroll_for<N, I + 1>(f);
+    }
+}
+
+// The same chains for many tokens: a K = 1 product per key steps every chain
+// of a wave's tile: R = 16 or 32 (token, head) rows -- 2 or 4 tokens' 8 heads
+// -- x 64 channels (v_mfma_f32_16x16x1_4b or 32x32x1_2b, its blocks side by
+// side over the channels).
+//
+// Both operands come straight from memory in the layout the product reads, no
+// LDS and no barrier: V as lane l's channel d0 + l of the key (one 256-byte
+// row piece a key), and the probabilities as lane (s, i) row i's keys 4 s ..
+// 4 s + 3 of a run, broadcast to every block by the product itself (CBSZ /
+// ABID: block s supplies operand A).  D batches of 16 keys are in flight.
+// (Staged through LDS for four 4x4x1 waves a block, the tile exchange and the
+// products added up instead of overlapping.)
+//
+// The tokens of a tile see the same keys but for a few at either end of their
+// ranges: there the product's result is kept only in the rows that see the
+// key, so every chain takes exactly its token's keys.
+template <int HD, int R, int D, bool FULL>
+__global__ __launch_bounds__(256) void k_attn_values(float *__restrict__ out, const float *__restrict__ probs,
+                                                     const float *__restrict__ value_cache, int cache_len,
+                                                     int start_pos, int n, size_t stride,
+                                                     int8_t *__restrict__ q8, float *__restrict__ qs) {
+    constexpr int TT = R / 8, B = 64 / R, KB = 16, PR = KB / (4 * B);  // PR runs of 4 B keys a batch
+    typedef float v4 __attribute__((ext_vector_type(4)));
+    typedef float vacc __attribute__((ext_vector_type(R)));
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // last tokens first: their rows are the longest
+    const int d0 = blockIdx.x * 64, t0 = ((gridDim.y - 1 - blockIdx.y) * 4 + wave) * TT;
+    if (t0 >= n) return;  // uniform per wave; no barrier
+    const int pos0 = start_pos + t0, pos_last = start_pos + min(t0 + TT, n) - 1;
+    // Batches start at multiples of 16 positions, so none wraps around the
+    // ring.  First the `head` ones that not every token of the tile sees from
+    // their first key on (a window's start), then `fast` ones whose keys all
+    // see, then the rest.
+    const int kfirst = first_visible(pos0, FULL) & ~(KB - 1), all_from = first_visible(pos_last, FULL);
+    const int batches = (pos_last - kfirst + KB) / KB, head = min((all_from - kfirst + KB - 1) / KB, batches);
+    const int fast = max((pos0 + 1 - kfirst) / KB - head, 0), whole = fast / D * D;
+
+    // Operands through buffer descriptors: scalar offsets, and what lies past
+    // the batch (a ring of fewer rows) or the tile's rows reads as 0 (never kept).
+    const int v_bytes = min(cache_len, KB) * HD * 4;
+    const __amdgpu_buffer_rsrc_t p_desc = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float *>(probs + (size_t)t0 * 8 * stride), 0,
+        (int)((uint32_t)min(R, (n - t0) * 8) * (uint32_t)stride * 4), 0x00020000);
+    const int i = lane % R, my_t = min(t0 + i / 8, n - 1), my_first = first_visible(start_pos + my_t, FULL);
+    const int my_last = start_pos + my_t - my_first;
+    const uint32_t my_row = (uint32_t)((my_t - t0) * 8 + i % 8) * (uint32_t)stride;
+    const int my_j = 4 * (lane / R) - my_first;
+    auto v_batch = [&](int k0) __attribute__((always_inline)) {
+        return __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<float *>(value_cache + (size_t)(k0 & (cache_len - 1)) * HD), 0, v_bytes, 0x00020000);
+    };
+    auto load_v = [&](__amdgpu_buffer_rsrc_t desc, auto e) __attribute__((always_inline)) {
+        return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                             desc, lane * 4, (decltype(e)::value * HD + d0) * 4, 0));
+    };
+    // run f's four probabilities of this lane (all_from on, so never before
+    // the row; without a window the run is 16-byte aligned and ends in the row)
+    auto load_p = [&](int k0, int f, float (&p)[4]) __attribute__((always_inline)) {
+        const uint32_t at = (my_row + (uint32_t)(k0 + 4 * B * f + my_j)) * 4;
+        if constexpr (FULL) {
+            const v4 x = __builtin_bit_cast(v4, __builtin_amdgcn_raw_buffer_load_b128(p_desc, at, 0, 0));
+            p[0] = x[0], p[1] = x[1], p[2] = x[2], p[3] = x[3];
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                p[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(p_desc, at + 4 * j, 0, 0));
+        }
+    };
+    vacc acc;
+#pragma unroll
+    for (int v = 0; v < R; v++) acc[v] = 0.0f;
+    auto product = [&](auto e, const float (&v)[KB], const float (&p)[PR][4]) __attribute__((always_inline)) {
+        constexpr int E = decltype(e)::value;
+        if constexpr (R == 16)
+            return __builtin_amdgcn_mfma_f32_16x16x1f32(p[E / 16][E % 4], v[E], acc, 2, E / 4 % 4, 0);
+        else
+            return __builtin_amdgcn_mfma_f32_32x32x1f32(p[E / 8][E % 4], v[E], acc, 1, E / 4 % 2, 0);
+    };
+    // a batch at either end: the product kept in the rows that see the key
+    auto masked = [&](int k0, const float (&v)[KB], const float (&p)[PR][4]) __attribute__((always_inline)) {
+        unroll_for<KB>([&](auto e) __attribute__((always_inline)) {
+            const int k = k0 + decltype(e)::value;
+            const vacc next = product(e, v, p);
+#pragma unroll
+            for (int x = 0; x < R; x++) {
+                // the token of output register x: of lanes 32 tt .. with 16
+                // rows, of registers 4 tt .. 4 tt + 3 (each block) with 32
+                const int pos = start_pos + t0 + (R == 16 ? lane / 32 : x / 4 % 4);
+                acc[x] = k >= first_visible(pos, FULL) && k <= pos ? next[x] : acc[x];
+            }
+        });
+    };
+    float vr[D][KB], pr[D][PR][4];
+    const int kfast = kfirst + head * KB;
+    unroll_for<D>([&](auto d) __attribute__((always_inline)) {
+        constexpr int S = decltype(d)::value;
+        const __amdgpu_buffer_rsrc_t desc = v_batch(kfast + S * KB);
+        unroll_for<KB>([&](auto e) __attribute__((always_inline)) { vr[S][decltype(e)::value] = load_v(desc, e); });
+#pragma unroll
+        for (int f = 0; f < PR; f++) load_p(kfast + S * KB, f, pr[S][f]);
+    });
+    // a batch with loads of its own, the probabilities clamped into the row
+    auto alone = [&](int k0) __attribute__((always_inline)) {
+        float v[KB], p[PR][4];
+        const __amdgpu_buffer_rsrc_t desc = v_batch(k0);
+        unroll_for<KB>([&](auto e) __attribute__((always_inline)) { v[decltype(e)::value] = load_v(desc, e); });
+#pragma unroll
+        for (int f = 0; f < PR; f++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const uint32_t at = my_row + (uint32_t)min(max(k0 + 4 * B * f + j + my_j, 0), my_last);
+                p[f][j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(p_desc, at * 4, 0, 0));
+            }
+        masked(k0, v, p);
+    };
+    for (int b = 0; b < head; b++) alone(kfirst + b * KB);
+    // the ring: each register refilled D batches ahead as soon as it is read,
+    // so that the loads and their addresses issue while the dependent products run
+    for (int b = 0; b < whole; b += D)
+        unroll_for<D>([&](auto d) __attribute__((always_inline)) {
+            constexpr int S = decltype(d)::value;
+            const int kn = kfast + (b + S + D) * KB;
+            const __amdgpu_buffer_rsrc_t desc = v_batch(kn);
+            unroll_for<KB>([&](auto e) __attribute__((always_inline)) {
+                constexpr int E = decltype(e)::value;
+                acc = product(e, vr[S], pr[S]);
+                __builtin_amdgcn_sched_barrier(0);
+                vr[S][E] = load_v(desc, e);
+                if constexpr ((E + 1) % (4 * B) == 0) load_p(kn, E / (4 * B), pr[S][E / (4 * B)]);
+                __builtin_amdgcn_sched_barrier(0);
+            });
+        });
+    // what is left, at most D + 1 batches: the first D are in the ring
+    const int rest = batches - head - whole;
+    unroll_for<D>([&](auto d) __attribute__((always_inline)) {
+        constexpr int S = decltype(d)::value;
+        if (S < rest) masked(kfast + (whole + S) * KB, vr[S], pr[S]);
+    });
+    for (int b = D; b < rest; b++) alone(kfast + (whole + b) * KB);
+
+    // output register x of block b: row 4 (l / 16) + x % 4 (16 rows), or
+    // 8 (x / 4 % 4) + 4 (l / 32) + x % 4 (32 rows); channel d0 + R b + l % R
+    constexpr int RB = R * R / 64;  // registers a block
+#pragma unroll
+    for (int x = 0; x < RB; x++) {
+        const int row = R == 16 ? 4 * (lane / 16) + x : 8 * (x / 4) + 4 * (lane / 32) + x % 4;
+        const int t = t0 + row / 8;
+        const size_t at = ((size_t)t * 8 + row % 8) * HD + d0 + lane % R;
+        if (!q8) {
+            if (t < n) {
+#pragma unroll
+                for (int b = 0; b < B; b++) out[at + R * b] = acc[RB * b + x];
+            }
+            continue;
+        }
+        // the o projection's input quantized here (k_quantize's arithmetic):
+        // the row's 64 channels are one group, R lanes x B registers
+        float m = 0.0f;
+#pragma unroll
+        for (int b = 0; b < B; b++) m = fmaxf(m, fabsf(acc[RB * b + x]));
+#pragma unroll
+        for (int o = R / 2; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
+        const float gscale = m / 127.0f, inverse = gscale > 0.0f ? 1.0f / gscale : 0.0f;
+        if (t < n) {
+#pragma unroll
+            for (int b = 0; b < B; b++) q8[at + R * b] = (int8_t)(int)rintf(acc[RB * b + x] * inverse);
+            if (lane % R == 0) qs[at / 64] = gscale;
+        }
+    }
+}
+
 // The row-local tail of the attention projections, one wave per row, in
 // reference order (gemma4.c:427-428 for the queries, 437-440 for a new key and
 // value): rmsnorm of each query head (q_norm) then RoPE in place; rmsnorm of
@@ -2420,14 +2680,14 @@ void launch_qkv_finish(hipStream_t s, float *q, int heads, const float *q_norm, 
 // probabilities are read through buffer descriptors.
 //   FULL (a global layer: keys 0 .. pos are cache rows 0 .. pos, no wrap):
 //   the V descriptor ends at row `keys`, so rows past the end read as 0.
-//   Sliding windows wrap around the ring; their keys are clamped to the last
-//   one (a valid row).
+//   Sliding windows wrap around the ring; keys past the end are read outside
+//   the descriptor, as 0.
 // V is prefetched DEPTH tiles ahead, the probabilities DEPTH - 1, in register
 // rings by unconditional loads (5 per tile, all countable by vmcnt; past the
-// end the probability loads reread the last tile).  The softmax writes 0 for
-// the keys between the row's end and its last whole tile, fma(0, v, o) = o
-// exactly (o is never -0, v finite or 0), and steps past the last tile skip
-// the chain.
+// end the probability loads reread the last tile).  The softmax writes -0 for
+// the keys between the row's end and its last whole tile, fma(-0, +0, o) = o
+// exactly (o = -0, infinite or NaN included), and steps past the last tile
+// skip the chain.
 
 template <int HD, int DEPTH, bool FULL, bool QUANT>
 __global__ __launch_bounds__(QUANT ? 256 : 64) void k_attn_values_decode(float *__restrict__ out,
@@ -2475,8 +2735,8 @@ __global__ __launch_bounds__(QUANT ? 256 : 64) void k_attn_values_decode(float *
         } else {
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-                const int key = min(tile * 64 + 4 * kq + i, keys - 1);
-                st.v[i] = load16(v_desc, (uint32_t)((first + key) & mask) * ROW + chan);
+                const int key = tile * 64 + 4 * kq + i;  // past the end: outside the descriptor
+                st.v[i] = load16(v_desc, key < keys ? (uint32_t)((first + key) & mask) * ROW + chan : 0xFFFFFF00u);
             }
         }
     };
@@ -2839,6 +3099,15 @@ int launch_attend_reference(hipStream_t s, float *out, const float *q, const flo
         return n > 4 && blocks > cap ? cap : blocks;
     };
     const unsigned nn = (unsigned)n;
+    // P V by the decode kernel (a wave per 16 channels x 4 heads, VALU chains of
+    // ~8 cycles a key) as long as its waves have a SIMD each or nearly: over a
+    // window 5 tokens 17 us for the layer's attention against 29, 64 tokens 24
+    // / 31, 100 30 / 32; 32 tokens over 6000 keys 146 / 190, 64 218 / 194.
+    // Rows of less than 256 keys are all prologue there: 37 tokens 13.2 / 12.2.
+    // 40 tokens of head dim 512 over 6000 keys 167 / 192, over 20000 624 / 610.
+    const bool few_values =
+        n <= 4 || (max_keys >= 256 && n * head_dim <= (max_keys <= 8192 ? 20480u : 16384u) &&
+                   (size_t)cache_len * head_dim < (size_t)1 << 29);  // (32-bit byte offsets)
     // Decode (at most 4 tokens) on the VALU kernel: 2 keys per 16-lane group
     // over the window, where the 512 keys then span 16 blocks instead of 8; 4
     // over a long context.  The matrix-core kernel's 32-row tiles would be
@@ -2866,22 +3135,28 @@ int launch_attend_reference(hipStream_t s, float *out, const float *q, const flo
         G4_SCORES(512, 1, 4);
     }
 #undef G4_SCORES
-    if (n <= 4) {  // decode: few rows, a block per row (the sum's block, when split)
+    // Rows: a block of 8-16 waves each while they are few (5 tokens over 6000
+    // keys: 81 us for the whole attention, 93 with four waves a row, 113 with
+    // one; 32 tokens 137 / 146 / 167; 64 222 / 218 / 240); one wave each where
+    // that makes several a SIMD (200 tokens over 6000 keys 316 against 306
+    // with four, but 512 602 / 641, over 1000 146 / 156).
+    if (n <= 4 || (few_values && n <= (max_keys <= G4_WINDOW ? 64u : 32u))) {  // (the sum's block, when split)
         const SoftmaxRows spec{heads, full, start_pos, 0, pos_dev, 1};
         if (split)
             launch_softmax_split(s, scores, stride, spec, (unsigned)(n * heads),
                                  reinterpret_cast<char *>(scores) + score_bytes);
         else
             launch_softmax_block(s, scores, stride, max_keys, spec, (unsigned)(n * heads));
-    } else if (max_keys <= 1024) {
-        hipLaunchKernelGGL(k_attn_softmax_reference<1>, dim3((unsigned)heads, nn), dim3(64), 0, s,
-                           scores, heads, full, start_pos, pos_dev, stride);
     } else {
-        hipLaunchKernelGGL(k_attn_softmax_reference<4>, dim3((unsigned)heads, nn), dim3(256), 0, s,
-                           scores, heads, full, start_pos, pos_dev, stride);
+        if (max_keys <= 1024 || n >= 384)
+            hipLaunchKernelGGL(k_attn_softmax_reference<1>, dim3((unsigned)heads, nn), dim3(64), 0, s, scores,
+                               heads, full, start_pos, stride, (int)few_values);
+        else
+            hipLaunchKernelGGL(k_attn_softmax_reference<4>, dim3((unsigned)heads, nn), dim3(256), 0, s, scores,
+                               heads, full, start_pos, stride, (int)few_values);
     }
     const unsigned slices = (unsigned)(head_dim / 64);
-    if (n <= 4) {  // decode: a wave per (16 channels, 4 heads, token), deep prefetch; with
+    if (few_values) {  // decode: a wave per (16 channels, 4 heads, token), deep prefetch; with
                    // q8 over a window, blocks of 4 such waves (64 channels) quantize their
                    // rows in place of the fp32 ones.  (Over a long context, four chains
                    // sharing a CU run at half speed: those waves keep a CU each and the
@@ -2913,16 +3188,35 @@ int launch_attend_reference(hipStream_t s, float *out, const float *q, const flo
 #undef G4_PV_DECODE
         if (q8 && !fuse) launch_quantize(s, q8, qs, out, n * heads * head_dim / 64);
         return G4_OK;
-    } else {  // prefill: 4 tokens x 8 heads per block share each V tile; one
-              // tile of prefetch (two or three measured no faster)
-        dim3 grid(slices, (nn + 3) / 4);
-        // with q8 the kernel writes the quantized rows (and no fp32 ones)
-        if (head_dim == 256)
-            hipLaunchKernelGGL((k_attn_values<256, 4, 1>), grid, dim3(256), 0, s, out, scores,
-                               value_cache, cache_len, full, start_pos, (int)n, pos_dev, stride, q8, qs);
-        else
-            hipLaunchKernelGGL((k_attn_values<512, 4, 1>), grid, dim3(256), 0, s, out, scores,
-                               value_cache, cache_len, full, start_pos, (int)n, pos_dev, stride, q8, qs);
+    } else {
+        // prefill; with q8 the kernels write the quantized rows (and no fp32
+        // ones).  Many tokens: k_attn_values, 4 waves a block on the same V; its
+        // 2-token waves have to fill the SIMDs (us for the whole attention,
+        // against the staged kernel): 512 tokens over 6000 keys 641 / 708, 200
+        // 306 / 365, 100 238 / 215; from position 0 (head dim 512) 54 / 58, but
+        // 256 over 556 keys 61 / 58 and 512 short windowed rows 46 / 44.  Its 4-token waves are half as many
+        // and gain only on long rows: over 7680 keys 750 / 776, 2000 274 / 262.
+        const bool many = n * head_dim >= 76800 && stride < (size_t)1 << 25 &&
+                          (head_dim == 256 ? start_pos >= 256 : max_keys >= (n >= 448 ? 384 : 640));
+        const bool wide = n * head_dim >= 230000 && max_keys >= 4096;
+#define G4_PV(HD, R, D, FULL)                                                                            \
+    hipLaunchKernelGGL((k_attn_values<HD, R, D, FULL>), dim3(slices, (nn + R / 2 - 1) / (R / 2)), dim3(256), 0, s, \
+                       out, scores, value_cache, cache_len, start_pos, (int)n, stride, q8, qs)
+#define G4_PV_STAGED(HD)                                                                              \
+    hipLaunchKernelGGL((k_attn_values_staged<HD, 4, 1>), dim3(slices, (nn + 3) / 4), dim3(256), 0, s, out, \
+                       scores, value_cache, cache_len, full, start_pos, (int)n, stride, q8, qs)
+        if (head_dim == 256) {
+            if (!many) G4_PV_STAGED(256);
+            else if (full) G4_PV(256, 16, 3, true);
+            else G4_PV(256, 16, 3, false);
+        } else {
+            if (!many) G4_PV_STAGED(512);
+            else if (!full) G4_PV(512, 16, 3, false);
+            else if (wide) G4_PV(512, 32, 4, true);
+            else G4_PV(512, 16, 3, true);
+        }
+#undef G4_PV_STAGED
+#undef G4_PV
         return G4_OK;
     }
 }

@@ -79,3 +79,40 @@ def test_prefill_attention_bitexact(pkg, g4lib, torch_gpu, oracle_lib, hd, ring,
         q[:] = 0.0
     o, ref = attend(pkg, g4lib, torch_gpu, oracle_lib, kc, vc, q, hd, ring, full, start, n)
     assert np.array_equal(o.view(np.uint32), ref.view(np.uint32)), int((o.view(np.uint32) != ref.view(np.uint32)).sum())
+
+
+# The routes of a pass by tokens and keys: the decode kernels for a few tokens
+# over long rows, staged tiles, two- and four-token waves for many; the first
+# and last count of each, with partial tiles, rings that wrap, and (inputs)
+# infinite values in the last visible row, NaN, and chains that underflow to -0.
+# head_dim, ring, full, start, tokens, inputs
+ROUTES = [
+    (256, 1024, 0, 251, 5, "special"), (256, 1024, 0, 250, 5, "normal"),     # max_keys 256, 255
+    (256, 1024, 0, 900, 80, "special"), (256, 1024, 0, 900, 81, "special"),
+    (512, 1024, 0, 300, 33, "special"), (512, 2048, 1, 1000, 40, "special"),
+    (512, 2048, 1, 1000, 41, "special"), (256, 8, 0, 0, 6, "normal"),        # a ring shorter than a batch
+    (256, 1024, 0, 256, 300, "special"), (256, 1024, 0, 255, 300, "normal"),
+    (256, 1024, 0, 5000, 301, "special"), (512, 2048, 0, 3000, 151, "special"),
+    (512, 2048, 1, 490, 150, "special"), (512, 1024, 1, 0, 449, "special"),
+    (256, 2048, 1, 256, 303, "special"), (512, 1024, 1, 489, 150, "normal"),
+    (512, 8192, 1, 3650, 451, "special"),                                     # four-token waves
+    (256, 512, 0, 0, 512, "special"),
+]
+
+
+@pytest.mark.parametrize("hd,ring,full,start,n,inputs", ROUTES)
+def test_attention_routes_bitexact(pkg, g4lib, torch_gpu, oracle_lib, hd, ring, full, start, n, inputs):
+    g = rng(4000 + hd + start + n)
+    kc = g.standard_normal((ring, hd)).astype(np.float32)
+    vc = g.standard_normal((ring, hd)).astype(np.float32)
+    q = (g.standard_normal((n, 8, hd)) * 0.25).astype(np.float32)
+    if inputs == "special":
+        last = (start + n - 1) & (ring - 1)
+        mid = (start + n // 2) & (ring - 1)
+        vc[last, 0::8], vc[mid, 1::8], vc[mid, 2::16] = np.inf, -np.inf, np.nan
+        vc[:, 3::8] = -np.abs(vc[:, 3::8]) * np.float32(2.0 ** -148)  # every product underflows to -0
+    with np.errstate(all="ignore"):
+        o, ref = attend(pkg, g4lib, torch_gpu, oracle_lib, kc, vc, q, hd, ring, full, start, n)
+    nan = np.isnan(ref)
+    assert np.array_equal(np.isnan(o), nan)
+    assert np.array_equal(o.view(np.int32)[~nan], ref.view(np.int32)[~nan])
