@@ -254,13 +254,21 @@ struct FixedScratch {
     void *ptr;
     size_t bytes;
 };
+// The tail of one token's attention projections for launch_attend to run
+// inside (launch_qkv_finish's work): q then holds the raw projection, the new
+// key and value (k_new null: an earlier layer's rings) go into the rings.
+struct QkvFinish {
+    const float *q_norm, *k_new, *v_new, *k_norm, *cosines, *sines;
+    int pairs;
+};
 // gemma4.c:443-456: attention over a ring cache; dispatches on order().
-// pos_dev requires reference order and n == 1.
+// pos_dev and finish require reference order and n == 1.
 // With q8 set, the output is also written quantized (k_quantize's groups).
 int launch_attend(hipStream_t s, float *out, const float *q, const float *key_cache,
                   const float *value_cache, int cache_len, int head_dim, int heads, int full,
                   int start_pos, const int *pos_dev, size_t n, int8_t *q8 = nullptr,
-                  float *qs = nullptr, const FixedScratch *fixed = nullptr);
+                  float *qs = nullptr, const FixedScratch *fixed = nullptr,
+                  const QkvFinish *finish = nullptr);
 // Scratch bytes launch_attend needs for n query rows (8 heads, head_dim <= 512)
 // whose last position is last_pos, in the current summation order.
 size_t attend_scratch_bytes(size_t n, int last_pos);
@@ -276,7 +284,7 @@ int launch_attend_reference(hipStream_t s, float *out, const float *q, const flo
                             const float *value_cache, int cache_len, int head_dim, int heads,
                             int full, int start_pos, const int *pos_dev, size_t n,
                             int8_t *q8 = nullptr, float *qs = nullptr,
-                            const FixedScratch *fixed = nullptr);
+                            const FixedScratch *fixed = nullptr, const QkvFinish *finish = nullptr);
 // Argument checks of g4_attend (shared by its allocation-free variant).
 int check_attend_args(const char *who, float *out, const float *q, const float *key_cache,
                       const float *value_cache, int cache_len, int head_dim, int heads,

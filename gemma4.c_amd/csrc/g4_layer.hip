@@ -116,7 +116,10 @@ extern "C" int g4_attention_layer(void *stream, float *hidden, size_t n, int sta
         G4_TRY(launch_matmul(s, b.aux, qw, b.q8, b.qs, (const int8_t *)q.data, q.scales, qw, G4_HIDDEN, (int)n));
     }
     // gemma4.c:427-428, 437-440: norms and RoPE, the new rows into the ring
-    if (order() == G4_ORDER_REFERENCE) {
+    const bool one = order() == G4_ORDER_REFERENCE && n == 1;  // (in the score kernel below)
+    const QkvFinish finish{qn, writes ? b.k_new : nullptr, b.v_new, kn, cs, sn, pairs};
+    if (one) {
+    } else if (order() == G4_ORDER_REFERENCE) {
         launch_qkv_finish(s, b.aux, 8, qn, writes ? b.k_new : nullptr, b.v_new, kn, keys, values, cs, sn,
                           pairs, hd, cache_len, start_pos, nullptr, n);
     } else {
@@ -128,7 +131,7 @@ extern "C" int g4_attention_layer(void *stream, float *hidden, size_t n, int sta
     }
     // gemma4.c:443-456, 459-460: attention, quantized for the output projection
     G4_TRY(launch_attend(s, b.att, b.aux, keys, values, cache_len, hd, 8, full_attention, start_pos,
-                         nullptr, n, b.q8, b.qs));
+                         nullptr, n, b.q8, b.qs, nullptr, one ? &finish : nullptr));
     G4_TRY(launch_matmul(s, hidden, G4_HIDDEN, b.q8, b.qs, (const int8_t *)o.data, o.scales, G4_HIDDEN,
                          qw, (int)n));
     G4_HIP(hipGetLastError());

@@ -653,7 +653,11 @@ static int enqueue_forward(Context &c, const Lane &ln, int n, int start_pos, con
                 G4_TRY(matmul(ln.v_new, hd, L.v, n));
             }
         }
-        if (fused) {  // query norms + RoPE and the new key/value rows: one launch
+        const QkvFinish finish{L.q_norm, L.k.data ? ln.k_new : nullptr, ln.v_new, L.k_norm,
+                               L.rope_cos, L.rope_sin, L.pairs};
+        if (one) {
+            // the query norms + RoPE and the new key/value rows: in the score kernel below
+        } else if (fused) {  // query norms + RoPE and the new key/value rows: one launch
             launch_qkv_finish(s, ln.aux, heads, L.q_norm, L.k.data ? ln.k_new : nullptr, ln.v_new,
                               L.k_norm, keys, values, L.rope_cos, L.rope_sin, L.pairs, hd, cache_len,
                               start_pos, pos_dev, n);
@@ -669,7 +673,7 @@ static int enqueue_forward(Context &c, const Lane &ln, int n, int start_pos, con
         if (L.k.data && ln.wait_kv) G4_HIP(hipStreamWaitEvent(s, ln.wait_kv[l], 0));
         if (L.k.data && ln.record_kv) G4_HIP(hipEventRecord(ln.record_kv[l], s));
         G4_TRY(launch_attend(s, ln.hidden, ln.aux, keys, values, cache_len, hd, heads, L.full,
-                             start_pos, pos_dev, n, ln.q8, ln.qs, ln.attn_scratch));
+                             start_pos, pos_dev, n, ln.q8, ln.qs, ln.attn_scratch, one ? &finish : nullptr));
         G4_TRY(matmul(ln.hidden, G4_HIDDEN, L.o, n));
 
         // feed-forward

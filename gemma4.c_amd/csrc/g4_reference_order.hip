@@ -1163,6 +1163,56 @@ __device__ __forceinline__ int first_visible(int pos, int full) {
     return !full && pos + 1 > G4_WINDOW ? pos + 1 - G4_WINDOW : 0;
 }
 
+// A row of the attention projections by one wave (gemma4.c:427-428, 437-440):
+// rmsnorm, then RoPE (not for a value).  Lane l holds elements J l .. J l +
+// J - 1 (J = HD / 64); the sum of squares is the sequential one
+// (wave_chain_sum), and element e's RoPE partner e + HD / 2 sits in lane l +
+// 32, same register.
+template <int HD>
+struct QkvRow {
+    static constexpr int J = HD / 64;
+    float x[J], w[J];
+    __device__ __forceinline__ void load(const float *src, const float *weight) {
+        const int lane = threadIdx.x & 63;
+#pragma unroll
+        for (int i = 0; i < J; i += 4) {
+            const float4 a = *reinterpret_cast<const float4 *>(src + J * lane + i);
+            const float4 b = weight ? *reinterpret_cast<const float4 *>(weight + J * lane + i)
+                                    : make_float4(1.0f, 1.0f, 1.0f, 1.0f);
+            x[i] = a.x, x[i + 1] = a.y, x[i + 2] = a.z, x[i + 3] = a.w;
+            w[i] = b.x, w[i + 1] = b.y, w[i + 2] = b.z, w[i + 3] = b.w;
+        }
+    }
+    // c, sn: the position's rows of the tables
+    __device__ __forceinline__ void finish(bool rope, const float *c, const float *sn, int pairs) {
+        const int lane = threadIdx.x & 63;
+        float sq[J];
+#pragma unroll
+        for (int i = 0; i < J; i++) sq[i] = x[i] * x[i];
+        const float inverse = 1.0f / sqrtf(wave_chain_sum<J>(sq) / (float)HD + 1e-6f);
+#pragma unroll
+        for (int i = 0; i < J; i++) x[i] = w[i] * (inverse * x[i]);
+        if (!rope) return;
+        const bool upper = lane >= 32;
+#pragma unroll
+        for (int i = 0; i < J; i++) {
+            const float other = __shfl_xor(x[i], 32);
+            const int jj = J * (lane & 31) + i;  // the pair index
+            if (jj < pairs) {
+                const float cj = c[jj], sj = sn[jj];
+                // first = element jj (lower lane), second = jj + HD / 2 (upper lane)
+                x[i] = upper ? x[i] * cj + other * sj : x[i] * cj - other * sj;
+            }
+        }
+    }
+    __device__ __forceinline__ void store(float *dst) const {
+        const int lane = threadIdx.x & 63;
+#pragma unroll
+        for (int i = 0; i < J; i += 4)
+            *reinterpret_cast<float4 *>(dst + J * lane + i) = make_float4(x[i], x[i + 1], x[i + 2], x[i + 3]);
+    }
+};
+
 // Lane l of each 16-lane row receives x from lane l + N of the same row
 // (DPP row_shl; lanes past the row's end receive 0).
 template <int N>
@@ -1308,6 +1358,108 @@ __global__ __launch_bounds__(256) void k_attn_scores(const float *__restrict__ q
                 const int v = (V / 16) * m + j, h = v / KG, p = kbase + k0 + v % KG;
                 if (p >= first && p <= pos) scores[((size_t)t * 8 + h) * stride + (p - first)] = x[j];
             }
+        }
+    }
+}
+
+// One token's scores with the tail of its projections inside (k_qkv_finish's
+// rows): every block norms and rotates the 8 query heads itself, two a wave,
+// its first keys already loading, into the same LDS rows; the block whose keys
+// include the token's own also finishes the new key and value, writes them
+// into the rings and takes that key from LDS.  One launch instead of two (a
+// decode step's layers: 4.5 + 3.9 us).
+template <int HD, int KG>
+__global__ __launch_bounds__(256) void k_attn_scores_decode(const float *__restrict__ q, QkvFinish f,
+                                                            float *key_cache, float *value_cache, int cache_len,
+                                                            int full, int start_pos,
+                                                            const int *__restrict__ pos_dev, size_t stride,
+                                                            float *__restrict__ scores) {
+    constexpr int S = HD / 16, SP = S + 4, KB = 16 * KG, J = HD / 64;
+    __shared__ __attribute__((aligned(16))) float s_q[8][16][SP];
+    __shared__ __attribute__((aligned(16))) float s_k[HD];
+    const int pos = pos_dev ? *pos_dev : start_pos, first = first_visible(pos, full);
+    const int blocks = gridDim.x, bx = blockIdx.x;
+    if (first + bx * KB > pos) return;
+    const int mask = cache_len - 1, lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int m = lane & 15, k0 = (wave * 4 + (lane >> 4)) * KG;
+    const bool owner = f.k_new && (pos - first) / KB % blocks == bx;
+    float kv[KG][S];
+    auto load_keys = [&](int kbase) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < KG; i++) {
+            const int p = min(kbase + k0 + i, pos);  // past the end: a valid row, not written
+            const float *kr = key_cache + (size_t)(p & mask) * HD + m;
+#pragma unroll
+            for (int s = 0; s < S; s++) kv[i][s] = kr[16 * s];
+        }
+    };
+    const float *c = f.cosines + (size_t)pos * f.pairs, *sn = f.sines + (size_t)pos * f.pairs;
+    QkvRow<HD> row[2], extra;
+#pragma unroll
+    for (int r = 0; r < 2; r++) row[r].load(q + (2 * wave + r) * HD, f.q_norm);
+    if (owner && wave < 2) extra.load(wave ? f.v_new : f.k_new, wave ? nullptr : f.k_norm);
+    if (HD == 256) load_keys(first + bx * KB);  // (128 registers with 512: after the rows)
+#pragma unroll
+    for (int r = 0; r < 2; r++) {
+        row[r].finish(true, c, sn, f.pairs);
+#pragma unroll
+        for (int i = 0; i < J; i++) {
+            const int e = J * lane + i;
+            s_q[2 * wave + r][e & 15][e >> 4] = row[r].x[i];
+        }
+    }
+    if (owner && wave < 2) {
+        extra.finish(!wave, c, sn, f.pairs);
+        extra.store((wave ? value_cache : key_cache) + (size_t)(pos & mask) * HD);
+        if (!wave) extra.store(s_k);
+    }
+    __syncthreads();
+    for (int kbase = first + bx * KB; kbase <= pos; kbase += blocks * KB) {
+        if (HD != 256 || kbase != first + bx * KB) load_keys(kbase);
+        if (owner && pos - kbase < KB) {  // the pass that holds the token's own key
+#pragma unroll
+            for (int i = 0; i < KG; i++)
+                if (kbase + k0 + i == pos) {
+#pragma unroll
+                    for (int s = 0; s < S; s++) kv[i][s] = s_k[16 * s + m];
+                }
+        }
+        if (kbase + k0 > pos) continue;  // uniform within the 16-lane group
+        float acc[8][KG];
+#pragma unroll
+        for (int h = 0; h < 8; h++)
+#pragma unroll
+            for (int i = 0; i < KG; i++) acc[h][i] = 0.0f;
+#pragma unroll
+        for (int s4 = 0; s4 < S / 4; s4++) {
+#pragma unroll
+            for (int h = 0; h < 8; h++) {
+                const float4 qq = reinterpret_cast<const float4 *>(s_q[h][m])[s4];
+#pragma unroll
+                for (int i = 0; i < KG; i++) {
+                    acc[h][i] = fmaf(qq.x, kv[i][4 * s4 + 0], acc[h][i]);
+                    acc[h][i] = fmaf(qq.y, kv[i][4 * s4 + 1], acc[h][i]);
+                    acc[h][i] = fmaf(qq.z, kv[i][4 * s4 + 2], acc[h][i]);
+                    acc[h][i] = fmaf(qq.w, kv[i][4 * s4 + 3], acc[h][i]);
+                }
+            }
+        }
+        // the reference's tree, as in k_attn_scores
+        constexpr int V = 8 * KG;
+        float x[V];
+#pragma unroll
+        for (int h = 0; h < 8; h++)
+#pragma unroll
+            for (int i = 0; i < KG; i++) x[h * KG + i] = acc[h][i];
+        butterfly_level<V, 8>(x, m);
+        butterfly_level<V / 2, 4>(x, m);
+        butterfly_level<V / 4, 2>(x, m);
+        butterfly_level<V / 8, 1>(x, m);
+#pragma unroll
+        for (int j = 0; j < V / 16; j++) {
+            const int v = (V / 16) * m + j, h = v / KG, p = kbase + k0 + v % KG;
+            if (p <= pos) scores[h * stride + (p - first)] = x[j];
         }
     }
 }
@@ -2592,9 +2744,7 @@ __global__ __launch_bounds__(256) void k_attn_values(float *__restrict__ out, co
 // the new key (k_norm) then RoPE, and the weightless rmsnorm of the new value,
 // both written into the rings at (start_pos + t) & (cache_len - 1).  Block
 // (r, t): r < heads a query head of token t, r = heads its key, heads + 1 its
-// value.  Lane l holds elements J l .. J l + J - 1 (J = HD / 64); the sum of
-// squares is the sequential one (wave_chain_sum), and element
-// e's RoPE partner e + HD / 2 sits in lane l + 32, same register.
+// value.
 template <int HD>
 __global__ __launch_bounds__(64) void k_qkv_finish(float *q, int heads, const float *__restrict__ q_norm,
                                                    const float *__restrict__ k_new,
@@ -2604,46 +2754,16 @@ __global__ __launch_bounds__(64) void k_qkv_finish(float *q, int heads, const fl
                                                    const float *__restrict__ sines, int pairs,
                                                    int cache_len, int start_pos,
                                                    const int *__restrict__ pos_dev) {
-    constexpr int J = HD / 64;
     if (pos_dev) start_pos = *pos_dev;
-    const int r = blockIdx.x, t = blockIdx.y, lane = threadIdx.x;
+    const int r = blockIdx.x, t = blockIdx.y;
     const int pos = start_pos + t;
     const bool is_q = r < heads, is_v = r == heads + 1;
     const float *src = is_q ? q + ((size_t)t * heads + r) * HD : (is_v ? v_new : k_new) + (size_t)t * HD;
-    const float *weight = is_q ? q_norm : is_v ? nullptr : k_norm;
-    float x[J], w[J], sq[J];
-#pragma unroll
-    for (int i = 0; i < J; i += 4) {
-        const float4 a = *reinterpret_cast<const float4 *>(src + J * lane + i);
-        const float4 b = weight ? *reinterpret_cast<const float4 *>(weight + J * lane + i)
-                                : make_float4(1.0f, 1.0f, 1.0f, 1.0f);
-        x[i] = a.x, x[i + 1] = a.y, x[i + 2] = a.z, x[i + 3] = a.w;
-        w[i] = b.x, w[i + 1] = b.y, w[i + 2] = b.z, w[i + 3] = b.w;
-    }
-#pragma unroll
-    for (int i = 0; i < J; i++) sq[i] = x[i] * x[i];
-    const float inverse = 1.0f / sqrtf(wave_chain_sum<J>(sq) / (float)HD + 1e-6f);
-#pragma unroll
-    for (int i = 0; i < J; i++) x[i] = w[i] * (inverse * x[i]);
-    if (!is_v) {
-        const bool upper = lane >= 32;
-        const float *c = cosines + (size_t)pos * pairs, *sn = sines + (size_t)pos * pairs;
-#pragma unroll
-        for (int i = 0; i < J; i++) {
-            const float other = __shfl_xor(x[i], 32);
-            const int jj = J * (lane & 31) + i;  // the pair index
-            if (jj < pairs) {
-                const float cj = c[jj], sj = sn[jj];
-                // first = element jj (lower lane), second = jj + HD / 2 (upper lane)
-                x[i] = upper ? x[i] * cj + other * sj : x[i] * cj - other * sj;
-            }
-        }
-    }
-    float *dst = is_q ? q + ((size_t)t * heads + r) * HD
-                      : (is_v ? value_cache : key_cache) + (size_t)(pos & (cache_len - 1)) * HD;
-#pragma unroll
-    for (int i = 0; i < J; i += 4)
-        *reinterpret_cast<float4 *>(dst + J * lane + i) = make_float4(x[i], x[i + 1], x[i + 2], x[i + 3]);
+    QkvRow<HD> row;
+    row.load(src, is_q ? q_norm : is_v ? nullptr : k_norm);
+    row.finish(!is_v, cosines + (size_t)pos * pairs, sines + (size_t)pos * pairs, pairs);
+    row.store(is_q ? q + ((size_t)t * heads + r) * HD
+                   : (is_v ? value_cache : key_cache) + (size_t)(pos & (cache_len - 1)) * HD);
 }
 
 void launch_qkv_finish(hipStream_t s, float *q, int heads, const float *q_norm, const float *k_new,
@@ -2660,6 +2780,44 @@ void launch_qkv_finish(hipStream_t s, float *q, int heads, const float *q_norm, 
         hipLaunchKernelGGL(k_qkv_finish<512>, grid, dim3(64), 0, s, q, heads, q_norm, k_new, v_new,
                            k_norm, key_cache, value_cache, cosines, sines, pairs, cache_len, start_pos,
                            pos_dev);
+}
+
+// A window row's probabilities (k_softmax_block's arithmetic) by one wave into
+// LDS, J consecutive values a lane, -0 past the row's end; keys <= 64 J, the
+// row's stride a multiple of 64.
+template <int J>
+__device__ __forceinline__ void softmax_row_lds(const float *x, int keys, float *out) {
+    const int at = J * (threadIdx.x & 63), limit = (keys + 63) & ~63;
+    float run_max = x[0], raw[J], val[J], t[J], m = -INFINITY;
+    if constexpr (J % 4 == 0) {
+#pragma unroll
+        for (int j = 0; j < J; j += 4) {
+            const float4 f = *reinterpret_cast<const float4 *>(x + min(at + j, limit - 4));
+            raw[j] = f.x, raw[j + 1] = f.y, raw[j + 2] = f.z, raw[j + 3] = f.w;
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < J; j++) raw[j] = x[min(at + j, limit - 1)];
+    }
+#pragma unroll
+    for (int j = 0; j < J; j++) {
+        val[j] = at + j > 0 && at + j < keys ? raw[j] : -INFINITY;  // v_0 is the starting maximum, not a term
+        m = fmaxf(m, val[j]);
+    }
+    const float incl = wave_max_scan(m);
+    float before = fmaxf(run_max, dpp_float<0x138, 0xf>(incl, -INFINITY));  // lanes below
+    run_max = fmaxf(run_max, __int_as_float(__builtin_amdgcn_readlane(__float_as_int(incl), 63)));
+    uint32_t fresh = 0;
+#pragma unroll
+    for (int j = 0; j < J; j++) {
+        const bool is_new = val[j] > before;
+        t[j] = is_new ? expf_libm(before - val[j]) : expf_libm(val[j] - before);
+        fresh |= (uint32_t)is_new << j;
+        before = fmaxf(before, val[j]);
+    }
+    const float sum = wave_chain_softmax<J>(t, fresh, 1.0f);
+#pragma unroll
+    for (int j = 0; j < J; j++) out[at + j] = at + j < keys ? expf_libm(raw[j] - run_max) / sum : -0.0f;
 }
 
 // P.V for one token (decode): one wave per block, four heads per wave.  Lane
@@ -2689,7 +2847,12 @@ void launch_qkv_finish(hipStream_t s, float *q, int heads, const float *q_norm, 
 // exactly (o = -0, infinite or NaN included), and steps past the last tile
 // skip the chain.
 
-template <int HD, int DEPTH, bool FULL, bool QUANT>
+// SOFTMAX (with QUANT): `probs` holds the scores; the block's four waves first
+// turn its four heads' rows into probabilities in LDS, a wave a row, the first
+// V tiles (a whole window) in flight.  One launch instead of two (a decode
+// step's window layers: 4.3 + 5.9 us).
+
+template <int HD, int DEPTH, bool FULL, bool QUANT, bool SOFTMAX>
 __global__ __launch_bounds__(QUANT ? 256 : 64) void k_attn_values_decode(float *__restrict__ out,
                                                                          const float *__restrict__ probs,
                                                                          const float *__restrict__ value_cache,
@@ -2697,7 +2860,9 @@ __global__ __launch_bounds__(QUANT ? 256 : 64) void k_attn_values_decode(float *
                                                                          const int *__restrict__ pos_dev,
                                                                          size_t stride, int8_t *__restrict__ q8,
                                                                          float *__restrict__ qs) {
+    static_assert(!SOFTMAX || (QUANT && !FULL), "the softmax of window rows");
     constexpr int WPB = QUANT ? 4 : 1;  // waves a block; each stages its own tiles
+    __shared__ __attribute__((aligned(16))) float s_p[4][SOFTMAX ? G4_WINDOW : 4];  // [head][key]
     __shared__ __attribute__((aligned(16))) float s_vw[WPB][2][16][68];  // [wave][slot][channel][position]
     if (pos_dev) start_pos = *pos_dev;
     const int wave = WPB > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
@@ -2741,7 +2906,10 @@ __global__ __launch_bounds__(QUANT ? 256 : 64) void k_attn_values_decode(float *
         }
     };
     auto load_p = [&](int tile) __attribute__((always_inline)) {
-        return load16(p_desc, p_lane + (uint32_t)min(tile, tiles - 1) * 256);
+        if constexpr (SOFTMAX)
+            return *reinterpret_cast<const f4 *>(&s_p[r][64 * min(tile, tiles - 1) + 4 * j]);
+        else
+            return load16(p_desc, p_lane + (uint32_t)min(tile, tiles - 1) * 256);
     };
     auto store_v = [&](int slot, const VTile &st) __attribute__((always_inline)) {
         float *row = &s_v[slot][4 * cc][kq];
@@ -2784,7 +2952,17 @@ __global__ __launch_bounds__(QUANT ? 256 : 64) void k_attn_values_decode(float *
 #pragma unroll
     for (int s = 0; s < DEPTH; s++) {
         load_v(s, v_ring[s]);
-        p_ring[s] = load_p(s);
+        if (!SOFTMAX) p_ring[s] = load_p(s);
+    }
+    if constexpr (SOFTMAX) {
+        const float *x = prows + wave * stride;
+        if (keys <= 64)
+            softmax_row_lds<1>(x, keys, s_p[wave]);
+        else if (keys <= 256)
+            softmax_row_lds<4>(x, keys, s_p[wave]);
+        else
+            softmax_row_lds<8>(x, keys, s_p[wave]);
+        __syncthreads();
     }
     store_v(0, v_ring[0]);
     load_v(DEPTH, v_ring[0]);
@@ -2800,9 +2978,10 @@ __global__ __launch_bounds__(QUANT ? 256 : 64) void k_attn_values_decode(float *
 #pragma unroll
         for (int i = 0; i < 16; i++) col[i] = src[i];
         store_v((tile + 1) & 1, next);
+        if (SOFTMAX) p = load_p(tile);
         load_v(tile + 1 + DEPTH, next);  // unconditional: past the end, valid memory
         if (tile < tiles) chain64(col, p);
-        p = load_p(tile + DEPTH);
+        if (!SOFTMAX) p = load_p(tile + DEPTH);
     };
     // The steps are written out (a dynamically indexed ring would live in
     // scratch memory).
@@ -3054,10 +3233,11 @@ __global__ __launch_bounds__(128) void k_attn_values_decode_pc(float *__restrict
 int launch_attend_reference(hipStream_t s, float *out, const float *q, const float *key_cache,
                             const float *value_cache, int cache_len, int head_dim, int heads,
                             int full, int start_pos, const int *pos_dev, size_t n, int8_t *q8,
-                            float *qs, const FixedScratch *fixed) {
+                            float *qs, const FixedScratch *fixed, const QkvFinish *finish) {
     if (!n) return G4_OK;
     if (heads != 8) return set_error(G4_ERR_ARG, "reference-order attention needs 8 query heads");
-    if (pos_dev && n != 1) return set_error(G4_ERR_ARG, "device-side positions are for one token");
+    if ((pos_dev || finish) && n != 1)
+        return set_error(G4_ERR_ARG, "device-side positions and raw projections are for one token");
     const int last_pos = start_pos + (int)n - 1;
     // Keys a row can see, at most (with a device-side position start_pos is the
     // largest one the launches serve).
@@ -3116,7 +3296,15 @@ int launch_attend_reference(hipStream_t s, float *out, const float *q, const flo
     hipLaunchKernelGGL((k_attn_scores<HD, TQ, KG>), dim3(key_blocks(TQ, 16 * KG), (nn + TQ - 1) / TQ), \
                        dim3(256), 0, s, q, key_cache, cache_len, full, start_pos, (int)n, pos_dev,  \
                        stride, scores)
-    if (n > 4) {
+    if (finish) {  // one token: its projections' tail inside
+        float *keys = const_cast<float *>(key_cache), *values = const_cast<float *>(value_cache);
+        if (head_dim == 256)
+            hipLaunchKernelGGL((k_attn_scores_decode<256, 2>), dim3(key_blocks(1, 32)), dim3(256), 0, s, q, *finish,
+                               keys, values, cache_len, full, start_pos, pos_dev, stride, scores);
+        else
+            hipLaunchKernelGGL((k_attn_scores_decode<512, 4>), dim3(key_blocks(1, 64)), dim3(256), 0, s, q, *finish,
+                               keys, values, cache_len, full, start_pos, pos_dev, stride, scores);
+    } else if (n > 4) {
         // many tokens: the matrix-core kernel, 4 tokens a block; about 512
         // blocks (two a CU), each striding over the rest of its key blocks
         const unsigned ty = (nn + 3) / 4;
@@ -3140,7 +3328,10 @@ int launch_attend_reference(hipStream_t s, float *out, const float *q, const flo
     // one; 32 tokens 137 / 146 / 167; 64 222 / 218 / 240); one wave each where
     // that makes several a SIMD (200 tokens over 6000 keys 316 against 306
     // with four, but 512 602 / 641, over 1000 146 / 156).
-    if (n <= 4 || (few_values && n <= (max_keys <= G4_WINDOW ? 64u : 32u))) {  // (the sum's block, when split)
+    // (With q8 set, the rows of 1-4 windowed tokens are left to the P V kernel.)
+    const bool inner_softmax = n <= 4 && q8 && !full;
+    if (inner_softmax) {
+    } else if (n <= 4 || (few_values && n <= (max_keys <= G4_WINDOW ? 64u : 32u))) {  // (the sum's block, when split)
         const SoftmaxRows spec{heads, full, start_pos, 0, pos_dev, 1};
         if (split)
             launch_softmax_split(s, scores, stride, spec, (unsigned)(n * heads),
@@ -3164,24 +3355,26 @@ int launch_attend_reference(hipStream_t s, float *out, const float *q, const flo
         const bool fuse = q8 && !full;
         const unsigned wpb = fuse ? 4u : 1u;
         dim3 grid((unsigned)(head_dim / 16) / wpb, 2, nn);
-#define G4_PV_DECODE(HD, FULL, QUANT)                                                                 \
-    hipLaunchKernelGGL((k_attn_values_decode<HD, 8, FULL, QUANT>), grid, dim3(64 * wpb), 0, s, out,   \
+#define G4_PV_DECODE(HD, QUANT, SOFTMAX)                                                              \
+    hipLaunchKernelGGL((k_attn_values_decode<HD, 8, false, QUANT, SOFTMAX>), grid, dim3(64 * wpb), 0, s, out, \
                        scores, value_cache, cache_len, full, start_pos, pos_dev, stride, q8, qs)
-#define G4_PV_DECODE_Q(HD, FULL)  \
-    if (fuse)                     \
-        G4_PV_DECODE(HD, FULL, true); \
-    else                          \
-        G4_PV_DECODE(HD, FULL, false)
+#define G4_PV_DECODE_Q(HD)              \
+    if (inner_softmax)                  \
+        G4_PV_DECODE(HD, true, true);   \
+    else if (fuse)                      \
+        G4_PV_DECODE(HD, true, false);  \
+    else                                \
+        G4_PV_DECODE(HD, false, false)
         // a global layer: the staging on a second wave of each block
 #define G4_PV_DECODE_PC(HD)                                                                        \
     hipLaunchKernelGGL((k_attn_values_decode_pc<HD, 8>), dim3((unsigned)(head_dim / 16), 2, nn),    \
                        dim3(128), 0, s, out, scores, value_cache, cache_len, start_pos, pos_dev, stride)
         if (head_dim == 256) {
             if (full) G4_PV_DECODE_PC(256);
-            else G4_PV_DECODE_Q(256, false);
+            else G4_PV_DECODE_Q(256);
         } else {
             if (full) G4_PV_DECODE_PC(512);
-            else G4_PV_DECODE_Q(512, false);
+            else G4_PV_DECODE_Q(512);
         }
 #undef G4_PV_DECODE_PC
 #undef G4_PV_DECODE_Q
@@ -3224,11 +3417,11 @@ int launch_attend_reference(hipStream_t s, float *out, const float *q, const flo
 int launch_attend(hipStream_t s, float *out, const float *q, const float *key_cache,
                   const float *value_cache, int cache_len, int head_dim, int heads, int full,
                   int start_pos, const int *pos_dev, size_t n, int8_t *q8, float *qs,
-                  const FixedScratch *fixed) {
+                  const FixedScratch *fixed, const QkvFinish *finish) {
     if (g_order == G4_ORDER_REFERENCE)
         return launch_attend_reference(s, out, q, key_cache, value_cache, cache_len, head_dim,
-                                       heads, full, start_pos, pos_dev, n, q8, qs, fixed);
-    if (pos_dev) return set_error(G4_ERR_ARG, "device-side positions need reference order");
+                                       heads, full, start_pos, pos_dev, n, q8, qs, fixed, finish);
+    if (pos_dev || finish) return set_error(G4_ERR_ARG, "device-side positions need reference order");
     const int rc = launch_attend_parallel(s, out, q, key_cache, value_cache, cache_len, head_dim,
                                           heads, full, start_pos, n, fixed);
     if (!rc && q8) launch_quantize(s, q8, qs, out, n * heads * head_dim / 64);
