@@ -947,6 +947,7 @@ template <int NW, bool NORM_IN, bool ADD, bool NORM_OUT>
 struct RowTail {
     static constexpr int J = kTailGroups / NW;
     static_assert(J * NW == kTailGroups, "NW divides 24");
+    static constexpr int kBarriers = (NORM_IN ? 1 : 0) + (NORM_OUT ? 1 : 0) + 2;  // of compute()
     float r[J], a[J], wi[J], wo[J];
     __device__ __forceinline__ void load(const RowTailJob &tj) {
         load_row_j<J>(tj.res_in, r);
@@ -988,18 +989,26 @@ struct RowTail {
     }
 };
 
-template <int EPI, int W, int TAIL>
-__global__ __launch_bounds__(64 * W * (EPI == EPI_PLAIN ? 1 : EPI == EPI_GELU_PAIR ? 8 : 4))
+// HELP = 1 (one tail wave a strip-matrix): as many waves again that only
+// stream.  A tail wave that issues more than a few of its own tiles first
+// starts its tail late, and the tiles left wait for the tail's end; a second
+// wave takes 12 of the strip's 24 groups, in flight beside the tail from the
+// tail's first barrier on (issued at once they hold up the tail's own loads:
+// a 37-token prompt and 16 tokens 39.2 ms without help, 39.9 with 16 groups
+// issued at once, 39.1 with 16 and 38.5 with 12 after the barrier).
+template <int EPI, int W, int TAIL, int HELP = 0>
+__global__ __launch_bounds__(64 * W * (1 + HELP) * (EPI == EPI_PLAIN ? 1 : EPI == EPI_GELU_PAIR ? 8 : 4))
 void k_gemv_tail(GemvJob job, RowTailJob tj) {
     constexpr int NM = EPI == EPI_GELU_PAIR ? 2 : 1, S = EPI == EPI_PLAIN ? 1 : 4, SM = NM * S;
-    constexpr int NW = W * SM, NG = kTailGroups / W;
-    static_assert(NG * W == kTailGroups, "W divides 24");
+    constexpr int NW = W * SM, NG = HELP ? 12 : kTailGroups / W;  // groups of a tail wave
+    static_assert(HELP ? W == 1 : NG * W == kTailGroups, "W divides 24");
     __shared__ __attribute__((aligned(16))) float s_row[1536], s_sq[1536];
     __shared__ int s_q8[384];
     __shared__ float s_qs[kTailGroups];
     __shared__ float s_d[SM][kTailGroups][16], s_c[SM][kTailGroups][16], s_e[NM][64];
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int sm = wave / W, wv = wave % W;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int sm = HELP ? wave % NW : wave / W, wv = HELP ? 0 : wave % W;
     int mi = EPI == EPI_GELU_PAIR ? sm / S : 0, strip = blockIdx.x * S + sm % S;
     if (EPI == EPI_PLAIN)
         while (mi + 1 < job.count && strip >= job.m[mi].strips) strip -= job.m[mi++].strips;
@@ -1009,43 +1018,66 @@ void k_gemv_tail(GemvJob job, RowTailJob tj) {
     const int row = 4 * (lane & 3) + 2 * b2 + b3;
     const uint4 *tiles = reinterpret_cast<const uint4 *>(mat.w + (size_t)strip * 16 * 1536) + lane;
     const uint16_t *wscale = mat.ws + (size_t)strip * kTailGroups * 16 + row;
-    // the tail's inputs first, then the first PRE of this wave's weight tiles,
-    // in flight while the tail runs (more would stall the wave at issue: the
-    // memory pipeline takes only so many requests, and the tail would then
-    // start after the tiles' data instead of beside it); the rest after it
-    constexpr int PRE = NG < 4 ? NG : 4;
-    RowTail<NW, TAIL != 3, TAIL != 3, TAIL != 2> tail;
-    tail.load(tj);
-    __builtin_amdgcn_sched_barrier(0);  // keep the tail's loads ahead of the tiles'
-    uint4 t[NG];
-    uint16_t wsr[NG];
-#pragma unroll
-    for (int u = 0; u < PRE; u++) {
-        t[u] = tiles[(size_t)(g0 + u) * 64];
-        wsr[u] = wscale[(g0 + u) * 16];
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    tail.compute(tj, s_row, s_sq, s_q8, s_qs);
-#pragma unroll
-    for (int u = PRE; u < NG; u++) {
-        t[u] = tiles[(size_t)(g0 + u) * 64];
-        wsr[u] = wscale[(g0 + u) * 16];
-    }
     // every group's dot first (their butterflies interleave), then the stores
-    int d[NG];
+    auto dots = [&](int g, const auto &t, const auto &wsr) __attribute__((always_inline)) {
+        constexpr int N = sizeof(wsr) / sizeof(wsr[0]);
+        int d[N];
 #pragma unroll
-    for (int u = 0; u < NG; u++) {
-        int dd[1];
-        const int xx[1] = {s_q8[(g0 + u) * 16 + chunk]};
-        gemv_group_dots<1>(t[u], xx, b2, b3, dd);
-        d[u] = dd[0];
-    }
-    if (lane < 16) {
-#pragma unroll
-        for (int u = 0; u < NG; u++) {
-            s_d[sm][g0 + u][row] = (float)d[u];
-            s_c[sm][g0 + u][row] = half_bits_to_float(wsr[u]) * s_qs[g0 + u];
+        for (int u = 0; u < N; u++) {
+            int dd[1];
+            const int xx[1] = {s_q8[(g + u) * 16 + chunk]};
+            gemv_group_dots<1>(t[u], xx, b2, b3, dd);
+            d[u] = dd[0];
         }
+        if (lane < 16) {
+#pragma unroll
+            for (int u = 0; u < N; u++) {
+                s_d[sm][g + u][row] = (float)d[u];
+                s_c[sm][g + u][row] = half_bits_to_float(wsr[u]) * s_qs[g + u];
+            }
+        }
+    };
+    using Tail = RowTail<NW, TAIL != 3, TAIL != 3, TAIL != 2>;
+    if (HELP && wave >= NW) {
+        constexpr int N = kTailGroups - NG;
+        static_assert(Tail::kBarriers > 1, "the first barrier: the tail's inputs have arrived");
+        __syncthreads();
+        uint4 t[N];
+        uint16_t wsr[N];
+#pragma unroll
+        for (int u = 0; u < N; u++) {
+            t[u] = tiles[(size_t)(NG + u) * 64];
+            wsr[u] = wscale[(NG + u) * 16];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 1; i < Tail::kBarriers; i++) __syncthreads();
+        dots(NG, t, wsr);
+    } else {
+        // the tail's inputs first, then the first PRE of this wave's weight
+        // tiles, in flight while the tail runs (more would stall the wave at
+        // issue: the memory pipeline takes only so many requests, and the tail
+        // would then start after the tiles' data instead of beside it); the
+        // rest after it
+        constexpr int PRE = NG < 4 ? NG : 4;
+        Tail tail;
+        tail.load(tj);
+        __builtin_amdgcn_sched_barrier(0);  // keep the tail's loads ahead of the tiles'
+        uint4 t[NG];
+        uint16_t wsr[NG];
+#pragma unroll
+        for (int u = 0; u < PRE; u++) {
+            t[u] = tiles[(size_t)(g0 + u) * 64];
+            wsr[u] = wscale[(g0 + u) * 16];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        tail.compute(tj, s_row, s_sq, s_q8, s_qs);
+#pragma unroll
+        for (int u = PRE; u < NG; u++) {
+            t[u] = tiles[(size_t)(g0 + u) * 64];
+            wsr[u] = wscale[(g0 + u) * 16];
+        }
+        dots(g0, t, wsr);
     }
     __syncthreads();
     const int tid = threadIdx.x;
@@ -1083,20 +1115,20 @@ int launch_gemv_tail(hipStream_t s, const GemvJob &job, int epi, const RowTailJo
         (tail != 3 && tj.res_out == tj.res_in))
         return set_error(G4_ERR_ARG, "fused tail product: bad shape");
     const unsigned blocks = (unsigned)(epi == EPI_PLAIN ? strips : job.m[0].strips / 4);
-#define G4_GT(E, WW, T)                                                                     \
+#define G4_GT(E, WW, T, H)                                                                  \
     if (epi == E && tail == T) {                                                            \
-        constexpr int SM_ = (E == EPI_PLAIN ? 1 : E == EPI_GELU_PAIR ? 8 : 4);              \
-        hipLaunchKernelGGL((k_gemv_tail<E, WW, T>), dim3(blocks), dim3(64 * WW * SM_), 0, s, job, tj); \
+        constexpr int SM_ = (E == EPI_PLAIN ? 1 : E == EPI_GELU_PAIR ? 8 : 4) * (1 + H);    \
+        hipLaunchKernelGGL((k_gemv_tail<E, WW, T, H>), dim3(blocks), dim3(64 * WW * SM_), 0, s, job, tj); \
         return G4_OK;                                                                       \
     }
     // q, k and v: 6 waves a strip (4 groups each); the GELU pair: 8 strip-
-    // matrices of one wave (24 groups); the per-layer-embedding gate: 4 strips
+    // matrices of one tail wave (12 groups) and one helper; the per-layer-embedding gate: 4 strips
     // of 2 waves (12 groups)
-    G4_GT(EPI_PLAIN, 6, 1)
-    G4_GT(EPI_PLAIN, 6, 2)
-    G4_GT(EPI_PLAIN, 6, 3)
-    G4_GT(EPI_GELU_PAIR, 1, 1)
-    G4_GT(EPI_GELU_MUL, 2, 2)
+    G4_GT(EPI_PLAIN, 6, 1, 0)
+    G4_GT(EPI_PLAIN, 6, 2, 0)
+    G4_GT(EPI_PLAIN, 6, 3, 0)
+    G4_GT(EPI_GELU_PAIR, 1, 1, 1)
+    G4_GT(EPI_GELU_MUL, 2, 2, 0)
 #undef G4_GT
     return set_error(G4_ERR_ARG, "fused tail product: no kernel for epilogue %d with tail %d", epi, tail);
 }
@@ -1399,7 +1431,7 @@ __global__ __launch_bounds__(256) void k_attn_scores_decode(const float *__restr
 #pragma unroll
     for (int r = 0; r < 2; r++) row[r].load(q + (2 * wave + r) * HD, f.q_norm);
     if (owner && wave < 2) extra.load(wave ? f.v_new : f.k_new, wave ? nullptr : f.k_norm);
-    if (HD == 256) load_keys(first + bx * KB);  // (128 registers with 512: after the rows)
+    if (HD == 256) load_keys(first + bx * KB);  // (with 512 no faster ahead of the rows)
 #pragma unroll
     for (int r = 0; r < 2; r++) {
         row[r].finish(true, c, sn, f.pairs);
@@ -3302,7 +3334,9 @@ int launch_attend_reference(hipStream_t s, float *out, const float *q, const flo
             hipLaunchKernelGGL((k_attn_scores_decode<256, 2>), dim3(key_blocks(1, 32)), dim3(256), 0, s, q, *finish,
                                keys, values, cache_len, full, start_pos, pos_dev, stride, scores);
         else
-            hipLaunchKernelGGL((k_attn_scores_decode<512, 4>), dim3(key_blocks(1, 64)), dim3(256), 0, s, q, *finish,
+            // 2 keys a group here too: a short context is one or two blocks, each half as
+            // long (37-token prompt and 16 tokens 39.5 -> 39.1 ms)
+            hipLaunchKernelGGL((k_attn_scores_decode<512, 2>), dim3(key_blocks(1, 32)), dim3(256), 0, s, q, *finish,
                                keys, values, cache_len, full, start_pos, pos_dev, stride, scores);
     } else if (n > 4) {
         // many tokens: the matrix-core kernel, 4 tokens a block; about 512
